@@ -876,9 +876,7 @@ int launch_flash_attention_blockwise(const FlashAttnDesc &d, hipStream_t s) {
         }
         return check_launch("flash_attention (fused)");
     }
-    const bool big_batch = d.batch > 16;
-    // 1. S = scale * Q . K^T  (per batch element when the single-GEMM tile
-    //    kernels fit, else one strided-batched call)
+    // 1. S = scale * Q . K^T
     auto gemm = [&](bool nt, const float *a, int64_t lda, int64_t sa, const float *b, int64_t ldb, int64_t sb,
                     float *c, int64_t ldc, int64_t sc, int64_t m, int64_t n, int64_t k, float alpha) -> int {
         SgemmDesc g;
@@ -893,15 +891,6 @@ int launch_flash_attention_blockwise(const FlashAttnDesc &d, hipStream_t s) {
         g.ldb = ldb;
         g.c = c;
         g.ldc = ldc;
-        if (!big_batch && sa % 4 == 0 && sb % 4 == 0 && sc % 4 == 0 && sgemm_big_fits(g)) {
-            for (int64_t bi = 0; bi < d.batch; ++bi) {
-                g.a = a + bi * sa;
-                g.b = b + bi * sb;
-                g.c = c + bi * sc;
-                GFH_TRY(launch_sgemm(g, s));
-            }
-            return GFH_SUCCESS;
-        }
         g.stride_a = sa;
         g.stride_b = sb;
         g.stride_c = sc;

@@ -1,11 +1,12 @@
 // gemm_nt_skinny.hip -- Linear::forward for a few rows of x:
-// y = alpha * x . W^T (+ beta y) (+ bias), x [m, k] with 4 < m <= 64 and W
+// y = alpha * x . W^T (+ beta y) (+ bias), x [m, k] with 4 < m <= 32 and W
 // [n, k] row-major, the reference's [out, in] weight
 // (ghostflow-nn/src/linear.rs:56-69) as gfh_sgemm's NT form.
 //
-// At these sizes the layer is HBM-bound up to m ~ 40 (every weight byte is
-// used m times) and no tile GEMM fills the GPU: a 64-row tile wastes most
-// of its MFMA rows and a grid of n / 64 workgroups cannot stream W.  So the
+// At these sizes the layer is HBM-bound (every weight byte is used m times)
+// and no tile GEMM streams W as fast (from 33 rows on sgemm_x3.hip's tiles
+// do: the fp32 SwiGLU 4096 x 11008 took 137 us here and 153 us there at 32
+// rows, 188 and 173 us at 48).  So the
 // weight is streamed from HBM straight into v_mfma_f32_16x16x4_f32
 // operands:
 //  * a workgroup owns 64 weight rows (output columns) over one K-slice;
@@ -29,8 +30,7 @@
 //    x is, and reads its MFMA fragments back with ds_read_b128.  Loaded
 //    straight into the fragments' registers, one instruction covered 16
 //    rows x 64 bytes (half lines); at [4096, 4096] the ring took 18.5 / 18.6
-//    / 21.8 / 30.6 us at m = 8 / 16 / 32 / 64 against 19.2 / 19.2 / 22.7 /
-//    34.3 us, the fp32 SwiGLU at m = 16 126.9 against 130.2 us, and three
+//    / 21.8 us at m = 8 / 16 / 32 against 19.2 / 19.2 / 22.7 us, the fp32 SwiGLU at m = 16 126.9 against 130.2 us, and three
 //    chunks ahead were slower than two (18.8 against 18.5 us at m = 8);
 //  * with fewer than ~512 workgroups K is also split over workgroups: each
 //    wave publishes its partial block with agent-scope stores and counts
@@ -90,9 +90,9 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 // MB: 16-row blocks of x (m <= 16 MB); D: chunks in flight ahead of the
 // MFMAs (D + 1 stages of each ring).  LDS: 12 KB x MB + 48 KB, so two
-// workgroups per CU up to 32 rows and one above.
+// workgroups per CU.
 template <int MB, int D>
-__global__ __launch_bounds__(64 * kWaves, MB <= 2 ? 2 : 1) void gemm_nt_skinny_kernel(SkNtParams p) {
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_nt_skinny_kernel(SkNtParams p) {
     constexpr int kXRows = 16 * MB;
     constexpr int kStageBytes = kXRows * kRowBytes;
     constexpr int kWStageBytes = kGroupCols * kRowBytes;
@@ -338,26 +338,21 @@ __global__ __launch_bounds__(64 * kWaves, MB <= 2 ? 2 : 1) void gemm_nt_skinny_k
 // K elements per workgroup: all of K with at least ~kTargetWgs workgroups
 // (or a batched call), otherwise enough slices for about that many, each at
 // least 4 chunks, a multiple of the chunk.  At [4096, 4096] (64 column
-// groups): 8 slices took 18.8 / 18.7 / 22.2 / 34.3 us at m = 8 / 16 / 32 /
-// 64, against 20.4-22.9 / 21.8-25.4 / 29-34 us with 4 and 21.3 / 27.2 /
-// 41.7 us (m = 8 / 32 / 64) with 16.  Of the 18.7 us at m = 16, about 2.7
+// groups): 8 slices took 18.8 / 18.7 / 22.2 us at m = 8 / 16 / 32,
+// against 20.4-22.9 / 21.8-25.4 / 29-34 us with 4 and 21.3 / 27.2 us (m = 8 /
+// 32) with 16.  Of the 18.7 us at m = 16, about 2.7
 // us are the split-K tail (partial stores, arrival count, the last
 // arriver's reads: three memory round trips) and 1 us the x staging.
-// Above 32 rows (three or four row blocks: one workgroup per CU, its LDS
-// rings 84-96 KB) half as many workgroups, one round of them: m = 40 / 48 /
-// 64 took 25.7 / 25.6 / 30.6 us against 28.5 / 28.9 / 34.3 us with the
-// weights in registers and 512 workgroups for m <= 48, while m <= 32
-// prefers 8 slices.
 constexpr int64_t kTargetWgs = 512;
 constexpr int kDepth = 2;
-// Up to 32 rows the slice count is rounded down: at N = 11008 (172 groups),
+// The slice count is rounded down: at N = 11008 (172 groups),
 // K = 4096, 2 slices took 45.9 / 46.8 / 56.8 us at m = 8 / 16 / 32 against
 // 49.9 / 50.3 / 57.4 with 3 (uneven: 1536, 1536, 1024 rows) and 57.6 /
 // 57.8 / 68.3 with none.
-int64_t choose_kslice(int64_t ngrp, int64_t k, int64_t batch, int64_t m) {
+int64_t choose_kslice(int64_t ngrp, int64_t k, int64_t batch) {
     const int64_t kc = ((k + kKC - 1) / kKC) * kKC;
     if (batch > 1) return kc;
-    int64_t s = m > 32 ? (kTargetWgs / 2 + ngrp - 1) / ngrp : kTargetWgs / ngrp;
+    int64_t s = kTargetWgs / ngrp;
     s = std::max<int64_t>(1, std::min<int64_t>(s, k / (4 * kKC)));
     const int64_t ks = (k + s - 1) / s;
     return (ks + kKC - 1) / kKC * kKC;
@@ -366,7 +361,7 @@ int64_t choose_kslice(int64_t ngrp, int64_t k, int64_t batch, int64_t m) {
 }  // namespace
 
 bool gemm_nt_skinny_fits(const SgemmDesc &d) {
-    return !d.trans_a && d.trans_b && d.m > kNtSkinnyMinM && d.m <= 64 && d.k > 0 && d.n > 0 && d.k % 4 == 0 &&
+    return !d.trans_a && d.trans_b && d.m > kNtSkinnyMinM && d.m <= 32 && d.k > 0 && d.n > 0 && d.k % 4 == 0 &&
            d.lda % 4 == 0 && d.ldb % 4 == 0 && aligned16(d.a) && aligned16(d.b) &&
            (d.batch_a <= 1 || d.stride_a % 4 == 0) && (d.batch_b <= 1 || d.stride_b % 4 == 0) && d.batch <= 65535;
 }
@@ -376,7 +371,7 @@ namespace {
 int launch_params(SkNtParams &p, int64_t gy, hipStream_t s) {
     const int64_t prods = p.ngroups > 0 ? p.ngroups : 1;
     p.ngrp = (p.n + kGroupCols - 1) / kGroupCols;
-    p.kslice = choose_kslice(p.ngrp * prods, p.k, p.ngroups > 0 ? 1 : gy, p.m);
+    p.kslice = choose_kslice(p.ngrp * prods, p.k, p.ngroups > 0 ? 1 : gy);
     p.slices = (p.k + p.kslice - 1) / p.kslice;
     if (p.slices > 1) {
         void *ws = nullptr;
@@ -387,12 +382,8 @@ int launch_params(SkNtParams &p, int64_t gy, hipStream_t s) {
     const dim3 grid((unsigned)(p.ngrp * p.slices), (unsigned)gy), block(64 * kWaves);
     if (p.m <= 16)
         hipLaunchKernelGGL((gemm_nt_skinny_kernel<1, kDepth>), grid, block, 0, s, p);
-    else if (p.m <= 32)
-        hipLaunchKernelGGL((gemm_nt_skinny_kernel<2, kDepth>), grid, block, 0, s, p);
-    else if (p.m <= 48)
-        hipLaunchKernelGGL((gemm_nt_skinny_kernel<3, kDepth>), grid, block, 0, s, p);
     else
-        hipLaunchKernelGGL((gemm_nt_skinny_kernel<4, kDepth>), grid, block, 0, s, p);
+        hipLaunchKernelGGL((gemm_nt_skinny_kernel<2, kDepth>), grid, block, 0, s, p);
     return check_launch("sgemm (NT skinny MFMA)");
 }
 }  // namespace

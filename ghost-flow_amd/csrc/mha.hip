@@ -80,9 +80,9 @@ int launch_mha_forward(const MhaDesc &d, void *workspace, hipStream_t s) {
     const SgemmDesc proj[3] = {linear_desc(d.query, d.b * d.sq, d.wq, d.bq, qbuf, e),
                                cache_desc(d.key, d.wk, d.bk, d.k_cache), cache_desc(d.value, d.wv, d.bv, d.v_cache)};
     const int nproj = d.sk > 0 ? 3 : 1;
-    // Up to 64 rows (the same rows of query, key and value) the three
-    // projections share one launch: 3x the columns fill the GPU better than
-    // one projection does, and two launch tails go away.
+    // Where query, key and value have the same rows the three projections
+    // share one launch: 3x the columns fill the GPU better than one projection
+    // does, and two launch tails go away.
     if (sgemm_nt_group_fits(proj, nproj)) {
         GFH_TRY(launch_sgemm_nt_group(proj, nproj, s));
     } else {

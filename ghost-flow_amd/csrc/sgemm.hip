@@ -274,12 +274,13 @@ int launch_variant(const SgemmParams &p, int64_t batch, hipStream_t s) {
 }  // namespace
 
 bool sgemm_nt_group_fits(const SgemmDesc *d, int count) {
-    return gemv_nt_group_fits(d, count) || gemm_nt_skinny_group_fits(d, count);
+    return gemv_nt_group_fits(d, count) || gemm_nt_skinny_group_fits(d, count) || sgemm_x3_group_fits(d, count);
 }
 
 int launch_sgemm_nt_group(const SgemmDesc *d, int count, hipStream_t s) {
     if (gemv_nt_group_fits(d, count)) return launch_gemv_nt_group(d, count, s);
     if (gemm_nt_skinny_group_fits(d, count)) return launch_gemm_nt_skinny_group(d, count, s);
+    if (sgemm_x3_group_fits(d, count)) return launch_sgemm_x3_group(d, count, s);
     return set_error(GFH_INVALID_SHAPE, "sgemm: these products do not share one launch");
 }
 
@@ -299,10 +300,10 @@ int launch_sgemm(const SgemmDesc &d, hipStream_t s) {
     // most of its MFMA rows empty and its grid far too small to stream W.
     if (gemv_nt_fits(d)) return launch_gemv_nt(d, s);
     if (gemv_nn_fits(d)) return launch_gemv_f32_epi(d.a, d.b, d.c, d.m, d.k, d.n, d.alpha, d.beta, d.bias, s);
-    // up to 64 rows: the weight streamed straight into f32 MFMA operands
+    // up to 32 rows: the weight streamed straight into f32 MFMA operands
     if (gemm_nt_skinny_fits(d)) return launch_gemm_nt_skinny(d, s);
-    // NT / NN on 256 x 256 tiles fed by direct-to-LDS loads, when they fill the GPU
-    if (sgemm_big_fits(d)) return launch_sgemm_big(d, s);
+    // everything else with K >= 32: bf16 pieces on the bf16 matrix units
+    if (sgemm_x3_fits(d)) return launch_sgemm_x3(d, s);
     SgemmParams p{};
     p.a = d.a;
     p.b = d.b;

@@ -66,8 +66,7 @@ size_t swiglu_f32_workspace_bytes(int64_t m, int64_t inter) {
 }
 
 // fp32: gate and up into the workspace, h over gate (or into d.h), then down.
-// Each product is a launch_sgemm NT call (gate and up as one grouped launch
-// when m <= 64).
+// Each product is a launch_sgemm NT call (gate and up as one grouped launch).
 int launch_swiglu_f32(const SwigluDesc &d, void *workspace, hipStream_t s) {
     const size_t one = round_up((size_t)d.m * (size_t)d.inter * 4);
     float *gate = static_cast<float *>(workspace);
@@ -88,8 +87,8 @@ int launch_swiglu_f32(const SwigluDesc &d, void *workspace, hipStream_t s) {
         g.bias = bias;
         return g;
     };
-    // Gate and up read the same x: up to 64 rows they share one grouped
-    // launch, otherwise one launch each.
+    // Gate and up read the same x and share one grouped launch (one launch
+    // each where no grouped kernel takes the shape).
     const SgemmDesc gu[2] = {linear(d.x, d.wg, d.bg, gate, d.inter, d.hidden),
                              linear(d.x, d.wu, d.bu, up, d.inter, d.hidden)};
     if (sgemm_nt_group_fits(gu, 2)) {

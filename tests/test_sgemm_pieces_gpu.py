@@ -1,0 +1,209 @@
+"""fp32 GEMM on bf16 pieces (sgemm_x3.hip): tile edges, cut-short K stages,
+layouts, unaligned rows, batches and K splits, and the values the pieces
+cannot carry (infinities, NaN, overflow, rows near the subnormals).
+
+Bar: with S = |A| |B| (the sum of the product magnitudes), each output is
+within (K/32 + 12) 2^-24 S of the exact one: one rounding of the running sum
+per 32 k, six per stage of the products, two for alpha / the K split, and
+under 2^-24 S left out of the products.
+"""
+import ctypes as C
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _gh():
+    import ghostflow_hip
+    return ghostflow_hip
+
+
+def _operands(torch, dev, m, n, k, ta, tb, seed, pad=0, scale=1.0):
+    """op(A) [m, k], op(B) [k, n] and the stored forms, `pad` floats between
+    rows and (with pad) a base 4 bytes off 16-byte alignment."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+
+    def stored(r, c):
+        ld = c + pad
+        buf = torch.randn(r * ld + 1, device=dev, generator=g) * scale
+        off = 1 if pad else 0
+        return buf, off, ld, buf[off:off + r * ld].view(r, ld)[:, :c]
+
+    a = stored(k, m) if ta else stored(m, k)
+    b = stored(n, k) if tb else stored(k, n)
+    opa = a[3].t() if ta else a[3]
+    opb = b[3].t() if tb else b[3]
+    return a, b, opa, opb
+
+
+def _sgemm(torch, gh, a, b, m, n, k, ta, tb, out, alpha=1.0, beta=0.0, bias=None):
+    L = gh.lib()
+    rc = L.gfh_sgemm(int(ta), int(tb), m, n, k, alpha, a[0].data_ptr() + 4 * a[1], a[2], b[0].data_ptr() + 4 * b[1],
+                     b[2], beta, out.data_ptr(), out.shape[1], None if bias is None else bias.data_ptr(),
+                     torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, L.gfh_last_error()
+
+
+def _check(torch, got, opa, opb, k):
+    ref = opa.double() @ opb.double()
+    s = opa.double().abs() @ opb.double().abs()
+    assert ((got.double() - ref).abs() <= (k / 32 + 12) * 2.0 ** -24 * s).all(), \
+        float(((got.double() - ref).abs() / s).max())
+
+
+# every tile size is reached: 32-row tiles (m <= 32), 64 x 64, 128 x 64,
+# 128 x 128 and 256 x 128, with remainders of rows, columns and K
+SHAPES = [(17, 70, 33), (32, 640, 1000), (40, 100, 63), (65, 129, 97), (64, 64, 32), (130, 257, 64), (500, 500, 95),
+          (1000, 700, 45), (700, 1500, 401), (2000, 1100, 129), (4100, 2050, 70), (96, 512, 4099)]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_edges_and_layouts(torch_dev, m, n, k, ta, tb):
+    import torch
+    gh = _gh()
+    for pad in (0, 3):
+        a, b, opa, opb = _operands(torch, torch_dev, m, n, k, ta, tb, m + n + k, pad)
+        out = torch.full((m, n + pad), 7.0, device=torch_dev)
+        _sgemm(torch, gh, a, b, m, n, k, ta, tb, out)
+        _check(torch, out[:, :n], opa, opb, k)
+        assert (out[:, n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(48, 192, 2048), (300, 260, 1056), (33, 64, 8190)])
+def test_epilogue_and_split_k(torch_dev, m, n, k):
+    """alpha, beta and bias on shapes whose K is split; three calls in a row
+    (the arrival counters return to zero) give the same bits."""
+    import torch
+    gh = _gh()
+    a, b, opa, opb = _operands(torch, torch_dev, m, n, k, 0, 1, k)
+    bias = torch.randn(n, device=torch_dev)
+    c0 = torch.randn(m, n, device=torch_dev)
+    plain = torch.empty(m, n, device=torch_dev)
+    _sgemm(torch, gh, a, b, m, n, k, 0, 1, plain)
+    _check(torch, plain, opa, opb, k)
+    want = (plain * 0.7 + c0 * -1.3) + bias
+    for _ in range(3):
+        out = c0.clone()
+        _sgemm(torch, gh, a, b, m, n, k, 0, 1, out, 0.7, -1.3, bias)
+        assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("m,n,k,ba,bb,batch", [(70, 50, 40, 6, 3, 6), (130, 300, 100, 5, 5, 5), (64, 65, 33, 1, 4, 4),
+                                               (300, 200, 65, 2, 1, 3)])
+def test_batches_modulo(torch_dev, m, n, k, ba, bb, batch):
+    import torch
+    gh = _gh()
+    for ta, tb in ((0, 0), (0, 1), (1, 0), (1, 1)):
+        a = torch.randn((ba,) + ((k, m) if ta else (m, k)), device=torch_dev)
+        b = torch.randn((bb,) + ((n, k) if tb else (k, n)), device=torch_dev)
+        out = torch.empty(batch, m, n, device=torch_dev)
+        rc = gh.lib().gfh_sgemm_strided_batched(ta, tb, m, n, k, 1.0, a.data_ptr(), a.shape[2], m * k, ba, b.data_ptr(),
+                                                b.shape[2], n * k, bb, 0.0, out.data_ptr(), n, m * n, batch, None,
+                                                torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        for i in range(batch):
+            x, y = a[i % ba], b[i % bb]
+            _check(torch, out[i], x.t() if ta else x, y.t() if tb else y, k)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+def test_whole_24_bits(torch_dev, ta, tb):
+    """A permutation matrix returns the other operand's bits: all three pieces
+    of every value arrive."""
+    import torch
+    gh = _gh()
+    n = 96
+    x = torch.randn(n, n, device=torch_dev) * torch.logspace(-20, 20, n, device=torch_dev)
+    perm = torch.eye(n, device=torch_dev)[torch.randperm(n, generator=torch.Generator().manual_seed(1)).to(torch_dev)]
+    for left in (True, False):
+        a, b = (perm, x) if left else (x, perm)
+        got = gh.sgemm(a.t().contiguous() if ta else a.contiguous(), b.t().contiguous() if tb else b.contiguous(),
+                       trans_a=bool(ta), trans_b=bool(tb))
+        idx = perm.argmax(1)
+        assert torch.equal(got, x[idx] if left else x[:, idx.argsort()])
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+def test_non_finite_values(torch_dev, tb):
+    """An infinity or NaN reaches exactly the outputs it reaches in fp32 (an
+    infinite term's sum is infinite, not NaN), and finite outputs stay within
+    the bound; sums that overflow give the infinity."""
+    import torch
+    gh = _gh()
+    m, n, k = 150, 140, 70
+    a = torch.randn(m, k, device=torch_dev)
+    b = torch.randn(k, n, device=torch_dev).abs() + 0.5
+    a[3, 5] = float("inf")
+    a[77, 9] = float("-inf")
+    a[140, 69] = float("nan")
+    a[20, :] = 3e38
+    a[21, :] = 3.4e38  # rounds up to infinity as a bf16
+    a[21, 1:] = 0.0
+    b[0, 100] = 0.25
+    got = gh.sgemm(a, b.t().contiguous() if tb else b, trans_b=bool(tb))
+    ref = a.double() @ b.double()
+    ref = torch.where(ref.abs() > 3.4028235677973366e38, ref.sign() * float("inf"), ref)
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got.isinf(), ref.isinf())
+    assert torch.equal(got[got.isinf()].double(), ref[ref.isinf()])
+    fin = ref.isfinite()
+    s = torch.nan_to_num(a.double().abs(), 0, 0, 0) @ b.double().abs()
+    assert ((got.double() - ref).abs()[fin] <= ((k / 2 + 12) * 2.0 ** -24 * s)[fin]).all()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+def test_tiny_rows(torch_dev, ta, tb):
+    """Rows whose low pieces would fall below the subnormals keep fp32
+    precision: against 64 bits, relative to S."""
+    import torch
+    gh = _gh()
+    m, n, k = 70, 66, 64
+    a, b, opa, opb = _operands(torch, torch_dev, m, n, k, ta, tb, 3)
+    opa.mul_(2.0 ** -118)
+    opb.mul_(2.0 ** 40)
+    opa[5:9].mul_(2.0 ** 100)
+    out = torch.empty(m, n, device=torch_dev)
+    _sgemm(torch, gh, a, b, m, n, k, ta, tb, out)
+    ref = opa.double() @ opb.double()
+    s = opa.double().abs() @ opb.double().abs()
+    # (the f32 chain: one rounding per 2 k)
+    assert ((out.double() - ref).abs() <= (k / 2 + 4) * 2.0 ** -24 * s).all()
+
+
+def test_group_equals_separate_products(torch_dev):
+    """The SwiGLU's gate and up share a launch: h from the block equals h from
+    separate linears within the bound carried through silu * up."""
+    import torch
+    gh = _gh()
+    m, hid, inter = 100, 192, 320
+    x = torch.randn(m, hid, device=torch_dev)
+    w = [torch.randn(inter, hid, device=torch_dev) * 0.1 for _ in range(2)]
+    bb = [torch.randn(inter, device=torch_dev) for _ in range(2)]
+    wd = torch.randn(hid, inter, device=torch_dev)
+    _, h = gh.swiglu(x, w[0], bb[0], w[1], bb[1], wd, None, want_h=True)
+    g, u = (x.double() @ wi.double().t() + bi.double() for wi, bi in zip(w, bb))
+    eps = (hid / 32 + 13) * 2.0 ** -24
+    sg, su = (x.double().abs() @ wi.double().abs().t() + bi.double().abs() for wi, bi in zip(w, bb))
+    ref = torch.nn.functional.silu(g) * u
+    bound = eps * (1.1 * sg * u.abs() + g.abs() * su) + 8 * 2.0 ** -24 * ref.abs() + 1e-30
+    assert ((h.double() - ref).abs() <= bound).all()
+
+
+def test_offset_limits_fall_back(torch_dev):
+    """A leading dimension beyond the tile kernel's 32-bit offsets still runs."""
+    import torch
+    gh = _gh()
+    ld, m, k, n = (1 << 21) + 8, 66, 40, 70
+    buf = torch.zeros((m - 1) * ld + k, device=torch_dev)
+    a = torch.as_strided(buf, (m, k), (ld, 1))
+    a.copy_(torch.randn(m, k, device=torch_dev))
+    b = torch.randn(k, n, device=torch_dev)
+    out = torch.empty(m, n, device=torch_dev)
+    rc = gh.lib().gfh_sgemm(0, 0, m, n, k, C.c_float(1.0), buf.data_ptr(), ld, b.data_ptr(), n, C.c_float(0.0),
+                            out.data_ptr(), n, None, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    s = a.double().abs() @ b.double().abs()
+    assert ((out.double() - a.double() @ b.double()).abs() <= (k + 4) * 2.0 ** -24 * s).all()
