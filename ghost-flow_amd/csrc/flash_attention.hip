@@ -494,7 +494,6 @@ __global__ __launch_bounds__(kFaThreads, 2) void fa_fused_kernel(FaFused p) {
 // buffer u % 3), all requested straight into LDS one tile ahead; 80 KB per
 // workgroup at d <= 128.
 //
-// Laid out as the balanced SDPA kernel:
 // 16-query sets on v_mfma_f32_16x16x4_f32, one set per wave, eight waves per
 // workgroup.  The query groups of a batch element (G = ceil(sq / 16)) are
 // paired as (G - 1 - p, p): waves 0-3 take the light groups p = 4 blockIdx.y

@@ -152,6 +152,9 @@ struct SdpaDesc {
     int64_t q_bs = 0, q_hs = 0, q_rs = 0, kv_bs = 0, kv_hs = 0, kv_rs = 0, o_bs = 0, o_hs = 0, o_rs = 0;
 };
 int launch_sdpa(const SdpaDesc &d, hipStream_t s);
+// attention_x3.hip: every call whose indices fit 32 bits.
+bool sdpa_x3_fits(const SdpaDesc &d);
+int launch_sdpa_x3(const SdpaDesc &d, hipStream_t s);
 
 // kv_attention.hip: a few queries over a K/V cache in [B, S, E] layout
 // (head h in columns h*d ..); strides in elements.
