@@ -38,8 +38,9 @@ const char *last_error();
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // ---- stream-ordered scratch ----------------------------------------------
-// Uses the caller's workspace when given (and large enough), otherwise
-// hipMallocAsync on the stream; releases with hipFreeAsync on destruction.
+// Uses the caller's workspace when given (and large enough), otherwise the
+// stream's kept block (up to 64 MB; released by gfh_shutdown), otherwise
+// hipMallocAsync on the stream, released with hipFreeAsync on destruction.
 class Scratch {
   public:
     Scratch() = default;
@@ -50,6 +51,7 @@ class Scratch {
   private:
     void *p_ = nullptr;
     bool owned_ = false;
+    int dev_ = -1;  // >= 0: p_ is the kept block of (dev_, s_)
     hipStream_t s_ = nullptr;
 };
 
