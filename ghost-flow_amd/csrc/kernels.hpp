@@ -39,6 +39,9 @@ bool gemm_nt_skinny_fits(const SgemmDesc &d);
 int launch_gemm_nt_skinny(const SgemmDesc &d, hipStream_t s);
 bool gemm_nt_skinny_group_fits(const SgemmDesc *d, int count);
 int launch_gemm_nt_skinny_group(const SgemmDesc *d, int count, hipStream_t s);
+// gate and up of a SwiGLU with silu(gate) * up written to h [m, n].
+bool gemm_nt_skinny_swiglu_fits(const SgemmDesc *gu);
+int launch_gemm_nt_skinny_swiglu(const SgemmDesc *gu, float *h, hipStream_t s);
 // sgemm.hip: up to kNtMaxGroups NT products of one shape in one launch
 // (whichever of the two forms above or sgemm_x3.hip serves m), or false / an
 // error when they do not fit one.

@@ -66,7 +66,8 @@ size_t swiglu_f32_workspace_bytes(int64_t m, int64_t inter) {
 }
 
 // fp32: gate and up into the workspace, h over gate (or into d.h), then down.
-// Each product is a launch_sgemm NT call (gate and up as one grouped launch).
+// Each product is a launch_sgemm NT call (gate and up as one grouped launch,
+// at 5-32 rows and wide layers with silu * up in its epilogue).
 int launch_swiglu_f32(const SwigluDesc &d, void *workspace, hipStream_t s) {
     const size_t one = round_up((size_t)d.m * (size_t)d.inter * 4);
     float *gate = static_cast<float *>(workspace);
@@ -91,13 +92,19 @@ int launch_swiglu_f32(const SwigluDesc &d, void *workspace, hipStream_t s) {
     // each where no grouped kernel takes the shape).
     const SgemmDesc gu[2] = {linear(d.x, d.wg, d.bg, gate, d.inter, d.hidden),
                              linear(d.x, d.wu, d.bu, up, d.inter, d.hidden)};
-    if (sgemm_nt_group_fits(gu, 2)) {
-        GFH_TRY(launch_sgemm_nt_group(gu, 2, s));
+    // (h inside x: gate and up must be finished before h is written)
+    const bool h_in_x = h < d.x + d.m * d.hidden && d.x < h + d.m * d.inter;
+    if (!h_in_x && gemm_nt_skinny_swiglu_fits(gu)) {
+        GFH_TRY(launch_gemm_nt_skinny_swiglu(gu, h, s));
     } else {
-        GFH_TRY(launch_sgemm(gu[0], s));
-        GFH_TRY(launch_sgemm(gu[1], s));
+        if (sgemm_nt_group_fits(gu, 2)) {
+            GFH_TRY(launch_sgemm_nt_group(gu, 2, s));
+        } else {
+            GFH_TRY(launch_sgemm(gu[0], s));
+            GFH_TRY(launch_sgemm(gu[1], s));
+        }
+        GFH_TRY(launch_silu_mul(gate, up, h, d.m * d.inter, s));
     }
-    GFH_TRY(launch_silu_mul(gate, up, h, d.m * d.inter, s));
     return launch_sgemm(linear(h, d.wd, d.bd, d.y, d.hidden, d.inter), s);
 }
 
