@@ -11,7 +11,9 @@ every input already resident in HBM.
 The same line carries
   * "roofline": the sgemm kernel's algorithmic FLOP per launch (2*M*N*K,
     bias excluded) over its average launch duration, timed with HIP events
-    on the stream the kernel runs on, against the f32 MFMA peak;
+    on the stream the kernel runs on, against the f32 MFMA peak (fp32
+    products on bf16 pieces run on the bf16 matrix units, so their fraction
+    of it can exceed 1: six bf16 products at 2.5 PFLOP/s are 417 TFLOP/s);
   * "cpu_baseline": the reference CPU path (the oracle's restatement of
     Linear::forward -> data_f32 gather of W^T + matmul_blocked + broadcast
     bias add, single-threaded as the reference is) timed on this host on a
