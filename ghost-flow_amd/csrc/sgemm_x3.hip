@@ -566,24 +566,30 @@ struct X3Plan {
     int slices;
 };
 
-// Tiles and what a stage of 32 k takes (us): one workgroup on an otherwise
-// idle CU of a part-filled launch, and per workgroup of a filled one (the
-// clock is lower there: the matrix units run at the power limit), plus a
-// tile's prologue and stores.  Fitted to 4096^3, 2048^3, 1024^3 and
-// 512-row products at K = 4096 and 11008 in every layout (within 10%).
+// Tiles and what they take (us): a stage of 32 k where a workgroup has its CU
+// to itself, the same per workgroup of a filled GPU (less where several share
+// a CU and hide each other's latency; more at 256x128 and 128x128, one per CU,
+// where the matrix units then run at the power limit), a tile's prologue and
+// stores; and how many of its workgroups share a CU.  Fitted to 4096^3,
+// 2048^3 and 110 products of 33-3000 rows, K 64-11008, N 128-11008 timed on
+// every tile and split: the choice is on average 1.1% slower than the fastest
+// of them.  (With every workgroup counted as a CU's only one, and without the
+// last arriver's reads below, 2.9%: 337 x 1152 x 1024 NN 22.5 us for 16.1,
+// 72 x 1702 x 3554 28.4 for 20.8.)
 struct X3Tile {
-    int bm, bn;
+    int bm, bn, per_cu;
     double alone, full, ends;
 };
-constexpr X3Tile kTiles[] = {{256, 128, 1.75, 2.30, 4.0},
-                             {128, 128, 1.00, 1.32, 2.5},
-                             {128, 64, 0.70, 0.75, 1.2},
-                             {64, 64, 0.46, 0.44, 0.6},
-                             {32, 64, 0.55, 0.29, 0.5}};
+constexpr X3Tile kTiles[] = {{256, 128, 1, 1.75, 2.20, 4.5},
+                             {128, 128, 1, 1.00, 1.32, 2.2},
+                             {128, 64, 2, 0.64, 0.71, 1.1},
+                             {64, 64, 3, 0.48, 0.44, 0.5},
+                             {32, 64, 4, 0.44, 0.30, 0.3}};
 
 // The tile and K split with the shortest estimated time for `count` products
-// of one shape: workgroups in rounds of one per CU, K slices (unless batched)
-// adding their partial tiles' traffic.
+// of one shape: workgroups in rounds of per_cu on every CU.  K slices (unless
+// batched) add the partial tiles' stores, at 6 TB/s, and the last arriver's
+// reads of a tile's partials, which one workgroup takes in at 100 GB/s.
 X3Plan plan_x3(const SgemmDesc &d, int64_t count, bool split) {
     const int64_t stages = (d.k + kBK - 1) / kBK;
     X3Plan best{0, 1};
@@ -591,14 +597,16 @@ X3Plan plan_x3(const SgemmDesc &d, int64_t count, bool split) {
     for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
         const X3Tile &t = kTiles[i];
         const int64_t tiles = ((d.m + t.bm - 1) / t.bm) * ((d.n + t.bn - 1) / t.bn) * count;
+        const int64_t round = (int64_t)t.per_cu * 256;
         for (int sl = 1; sl <= (split ? 16 : 1); ++sl) {
-            const double part = (double)sl * (double)tiles * t.bm * t.bn * 4;
+            const double one = (double)t.bm * t.bn * 4, part = (double)sl * (double)tiles * one;
             if (sl > 1 && (stages / sl < 4 || part > 64e6)) break;
-            const int64_t tasks = tiles * sl, rem = tasks % 256;
+            const int64_t tasks = tiles * sl, rem = tasks % round;
             const double st = (double)((stages + sl - 1) / sl);
-            double us = (double)(tasks / 256) * (st * t.full + t.ends);
-            if (rem) us += st * (rem <= 192 ? t.alone : t.full) + t.ends;
-            if (sl > 1) us += 2.5 + 2 * part / 6e6;
+            auto shared = [&](double n) { return std::max(st * t.alone, n * st * t.full) + n * t.ends; };
+            double us = (double)(tasks / round) * shared(t.per_cu);
+            if (rem) us += rem <= 192 ? st * t.alone + t.ends : shared((double)((rem + 255) / 256));
+            if (sl > 1) us += 2.5 + part / 6e6 + sl * one / 1e5;
             if (us < least) {
                 least = us;
                 best = {i, sl};

@@ -72,7 +72,8 @@ def test_edges_and_layouts(torch_dev, m, n, k, ta, tb):
         assert (out[:, n:] == 7.0).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(48, 192, 2048), (300, 260, 1056), (33, 64, 8190)])
+@pytest.mark.parametrize("m,n,k", [(48, 192, 2048), (300, 260, 1056), (33, 64, 8190), (700, 1700, 5000),
+                                   (130, 1579, 4515), (84, 960, 3520)])
 def test_epilogue_and_split_k(torch_dev, m, n, k):
     """alpha, beta and bias on shapes whose K is split; three calls in a row
     (the arrival counters return to zero) give the same bits."""
