@@ -14,7 +14,8 @@
 //   * causal masking is j > i -> -inf (ops.rs:205-224); an explicit mask is
 //     cycled over the flattened scores, m > 0.5 keeps (attention.rs:51-64);
 //   * a row whose scores are all -inf yields NaN, as softmax over all -inf
-//     does in the reference (max = -inf, exp(NaN)).
+//     does in the reference (max = -inf, exp(NaN)), and so does a row with a
+//     kept NaN score (its exponential enters the row's sum).
 //
 // Nearly every call runs on bf16 pieces (attention_x3.hip, where the figures
 // are); sdpa_fwd_kernel here takes those whose indices do not fit 32 bits.
@@ -189,9 +190,9 @@ __global__ __launch_bounds__(kThreads, 2) void sdpa_fwd_kernel(SdpaParams p) {
             tile_scores<DMAX, CAUSAL, MASK>(p, lk + cur * kTile, qf, k0, my_q, lane, sv);
             float mb = sv[0];
 #pragma unroll
-            for (int r = 1; r < 16; ++r) mb = fmaxf(mb, sv[r]);
-            mb = fmaxf(mb, __shfl_xor(mb, 32));
-            const float m_new = fmaxf(m, mb);
+            for (int r = 1; r < 16; ++r) mb = max_nan(mb, sv[r]);
+            mb = max_nan(mb, __shfl_xor(mb, 32));
+            const float m_new = max_nan(m, mb);
             const bool dead = (m_new == -INFINITY);  // every score so far masked
             const float alpha = dead ? 1.f : __expf(m - m_new);
             float psum = 0.f;

@@ -84,9 +84,6 @@ struct Tile {
     static constexpr bool kAll = kUnits % kThreads == 0;
 };
 
-// NaN-propagating maximum.
-__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
-
 // A thread's share of a K/V tile in registers.
 template <int DP>
 struct KvRegs {
@@ -149,13 +146,6 @@ constexpr float kBig = 0x1p60f;  // the pieces' range, with slack for the produc
 
 constexpr float kLog2e = 0x1.715476p+0f;
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
-
-__device__ __forceinline__ float quarter_max_nan(float x) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = max_nan(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return max_nan(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
 
 // Whether the mask keeps key `key` (< skv) for a query whose first flattened
 // score is `base` (reduced modulo mask_numel when mask_rows).
@@ -241,7 +231,7 @@ __device__ __forceinline__ void set_f32(const X3Attn &p, const float *Q, const f
     const int end = CAUSAL ? min(p.skv, q0 + 16 + p.off) : p.skv;
     for (int k0 = 0; k0 < end; k0 += 16) {
         f32x4 s = score(k0);
-        const float m_new = fmaxf(m, quarter_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+        const float m_new = max_nan(m, quarter_max_nan(max_nan(max_nan(s[0], s[1]), max_nan(s[2], s[3]))));
         const bool dead = m_new == -INFINITY;
         const float alpha = dead ? 1.f : __expf(m - m_new);
         float sum = 0.f;

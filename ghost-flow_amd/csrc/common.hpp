@@ -176,6 +176,10 @@ __device__ __forceinline__ float half_wave_sum(float v) {
     return (threadIdx.x & 32) ? hi : lo;
 }
 
+// NaN-propagating maximum: a running maximum of scores has to keep a NaN, or
+// one that starts at -infinity takes a row of NaN for a fully masked one.
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
 // ---- four lanes c, c + 16, c + 32, c + 48 -----------------------------------
 //
 // In the 16x16x4 MFMA layouts (lane l holds column l % 16 in quarter l / 16)
@@ -184,11 +188,11 @@ __device__ __forceinline__ float half_wave_sum(float v) {
 // v_permlane32_swap pairs it with l ^ 32 (both halves of each result hold
 // the two values), VALU ops instead of LDS-path permutes.  Every lane of the
 // four ends with the same result.
-__device__ __forceinline__ float quarter_max(float x) {
+__device__ __forceinline__ float quarter_max_nan(float x) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    x = max_nan(__uint_as_float(a[0]), __uint_as_float(a[1]));
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    return max_nan(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 __device__ __forceinline__ float quarter_sum(float x) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);

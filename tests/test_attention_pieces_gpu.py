@@ -178,3 +178,55 @@ def test_many_slices(torch_dev):
     b, h = 1 << 12, 1 << 11
     q, k, v = (torch.randn(b, h, 1, 4, device=torch_dev) for _ in range(3))
     assert torch.equal(gh.sdpa(q, k, v), v)
+
+
+@pytest.mark.parametrize("d", [20, 64, 128])
+@pytest.mark.parametrize("weights", [False, True])
+def test_nan_scores_reach_their_rows(torch_dev, weights, d):
+    """A kept NaN score makes its whole row NaN (the reference's maximum ignores
+    it, the sum of the row does not), also where every score before it, or the
+    whole first key tile, is NaN; a masked one leaves its row alone."""
+    import torch
+    gh = _gh()
+    s = 70
+    q, k, v = (torch.randn(1, 2, s, d, device=torch_dev) for _ in range(3))
+
+    def run(kk, **kw):
+        r = gh.sdpa(q, kk, v, want_weights=weights, **kw)
+        return r if weights else (r, r)
+
+    for first in (16, 32, 40):
+        bad = k.clone()
+        bad[0, 0, :first] = math.nan
+        for causal in (False, True):
+            clean = run(k, causal=causal)
+            for x, c in zip(run(bad, causal=causal), clean):
+                assert x[0, 0].isnan().all()
+                torch.testing.assert_close(x[0, 1], c[0, 1], rtol=0, atol=1e-5)
+    # of the first 16 keys, rows 10 .. 19 keep the NaN one alone and rows
+    # 20 .. 29 none of the NaN ones
+    bad = k.clone()
+    bad[0, 0, 3] = math.nan
+    mask = torch.ones(s, s, device=torch_dev)
+    mask[10:20, :16] = 0.0
+    mask[10:20, 3] = 1.0
+    mask[20:30, 3] = 0.0
+    rows = torch.zeros(s, dtype=torch.bool, device=torch_dev)
+    rows[20:30] = True
+    for x, c in zip(run(bad, mask=mask), run(k, mask=mask)):
+        assert x[0, 0, ~rows].isnan().all()
+        torch.testing.assert_close(x[0, 0, rows], c[0, 0, rows], rtol=0, atol=1e-5)
+
+
+def test_nan_scores_many_slices(torch_dev):
+    """The same in the kernel for 2^23 and more (batch, head) slices."""
+    import torch
+    gh = _gh()
+    b, h, skv, d = 1 << 12, 1 << 11, 40, 4
+    q, k, v = (torch.empty(b, h, n, d, device=torch_dev).normal_() for n in (1, skv, skv))
+    k[7, 9, :32] = math.nan
+    for weights in (False, True):
+        r = gh.sdpa(q, k, v, want_weights=weights)
+        for x in r if weights else (r,):
+            assert x[7, 9].isnan().all()
+            assert x[7, 8].isfinite().all() and x[7, 10].isfinite().all()
