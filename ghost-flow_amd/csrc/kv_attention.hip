@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_attention_kernel(KvParams p)
                 if (WEIGHTS && head_ok && lane == 0 && j < j1 && i < nq)
                     __hip_atomic_store(p.weights + (bh * p.sq + qi) * p.kv_len + j, s, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT);
-                const float m_new = fmaxf(m[i], s);
+                const float m_new = max_nan(m[i], s);
                 if (m_new == -INFINITY) continue;  // every key so far masked (uniform over the half-wave)
                 const float corr = __expf(m[i] - m_new);
                 const float pj = __expf(s - m_new);
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_attention_kernel(KvParams p)
 #pragma unroll
                     for (int g = 0; g < kG; ++g) {
                         if (sp0 + g >= p.nsplit || ms[g] == -INFINITY) continue;  // nothing kept in that split
-                        const float M_new = fmaxf(M, ms[g]);
+                        const float M_new = max_nan(M, ms[g]);
                         const float fo = __expf(M - M_new), fn = __expf(ms[g] - M_new);  // exp(-inf) = 0
                         L = L * fo + ls[g] * fn;
                         A = A * fo + as[g] * fn;

@@ -136,3 +136,26 @@ def test_decode_step_llama_shape(torch_dev):
     ref, _ = _ref(q, kc, vc, kv_len, h)
     got = to_np(gh.kv_attention(to_dev(q, torch_dev), to_dev(kc, torch_dev), to_dev(vc, torch_dev), kv_len, h))
     assert_rel(got, ref)
+
+
+@pytest.mark.parametrize("sq,kv_len,first", [(1, 5, 1), (2, 40, 20), (1, 3000, 1), (1, 3000, 2000), (3, 600, 64)])
+def test_nan_scores_reach_their_rows(torch_dev, sq, kv_len, first):
+    """A kept NaN score makes its row NaN, as the oracle's row sum does, also
+    where every key before it, or a whole split of the cache, is NaN; a masked
+    one leaves its row alone."""
+    gh = _gh()
+    b, h, d = 2, 3, 64
+    q, kc, vc = _case(b, h, d, sq, kv_len, kv_len + 1, seed=kv_len + first)
+    kc[0, :first, :d] = np.nan  # head 0 of element 0
+    mask = np.ones((b, h, sq, kv_len), np.float32)
+    mask[0, 0, sq - 1, :first] = 0.0
+    for mk in (None, mask):
+        ref, ref_w = _ref(q, kc, vc, kv_len, h, mask=mk)
+        got, w = gh.kv_attention(to_dev(q, torch_dev), to_dev(kc, torch_dev), to_dev(vc, torch_dev), kv_len, h,
+                                 mask=None if mk is None else to_dev(mk, torch_dev), want_weights=True)
+        got, w = to_np(got), to_np(w)
+        # (a masked NaN key times a weight of 0 stays out of the weights)
+        assert np.array_equal(np.isnan(w), np.isnan(ref_w)) and np.isnan(ref_w[0, 0]).any() == (mk is None or sq > 1)
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        assert_rel(np.nan_to_num(got), np.nan_to_num(ref))
+        assert_rel(np.nan_to_num(w), np.nan_to_num(ref_w))
