@@ -13,8 +13,8 @@
 // _bf16 per 32 k do the same product: a register-only loop of them on split
 // N(0, 1) data sustains 1920 TFLOP/s (320 of fp32 product; 1570 with the
 // 32x32x16 form) at about 1.8 GHz, the power limit.  Measured, before -> now
-// (us; NT / NN / TN): 4096^3 935 / 950 / 951 -> 587 / 597 / 621; 2048^3 NN
-// 131 -> 90; 1000 x 1500 x 784 NN 42.6 -> 24; 64 x 11008 x 4096 NT 90 -> 50.
+// (us; NT / NN / TN): 4096^3 935 / 950 / 951 -> 594 / 598 / 618; 2048^3 NN
+// 131 -> 93; 1000 x 1500 x 784 NN 42.6 -> 24.5; 64 x 11008 x 4096 NT 90 -> 56.
 // Relative error against 64 bits: 4096^3 1.1e-6 -> 2.2e-7, 512 x 512 x 64
 // 1.1e-7 -> 4.7e-8 (no shape of the sweep came out larger than before).
 //
@@ -44,8 +44,13 @@
 //    columns of C and stores them as one 16-byte store.
 //  * 74% of all cycles are MFMA-busy at 4096^3 (1.82 GHz); wider prefetch
 //    (2 and 4 stages) and a 2 x 4 wave grid measured the same.
-//  * Infinities, NaN, sums that overflow and rows below 2^-95 are computed
-//    again on the f32 instructions (sgemm_x3_kernel's end).
+//  * Both operands are scaled by 2^16 before they are split, so that every
+//    fp32 value down to the subnormals keeps its 24 bits beside elements of
+//    any size (unscaled, an element below 2^-110 lost its low bits, and rows
+//    and columns of such values had to be found and redone); the sums are
+//    scaled back at the end of K.  Infinities, NaN, elements of 2^112 and
+//    sums of 2^96 and more are computed again on the f32 instructions
+//    (sgemm_x3_kernel's end).
 #include <algorithm>
 
 #include "common.hpp"
@@ -100,8 +105,8 @@ struct X3Params {
     int *counters;
 };
 
-// Position of row r of chunk c among its 16-row block.
-__device__ __forceinline__ int spread(int r, int c) { return (r & ~15) | ((r & 15) ^ (c & 1 ? 14 : 0) ^ (c & 2 ? 4 : 0)); }
+// Row r of chunk c sits at r ^ swz(c) of its 16-row block.
+__device__ __forceinline__ constexpr int swz(int c) { return (c & 1 ? 14 : 0) ^ (c & 2 ? 4 : 0); }
 
 // One operand's share of a stage in registers.
 template <int R, int NT, bool KC>
@@ -113,12 +118,20 @@ struct X3Loader {
     static constexpr int U = R * (kBK / F) / NT;
     static_assert(U >= 1 && U * NT * F == R * kBK, "whole units per thread");
     float v[U][F];
-    uint32_t seen[U];   // OR of the unit's leading pieces, over all stages
-    uint32_t off[U];    // byte offset of the unit, from one stage before the one it is loaded from
+    uint32_t off[U];  // byte offset of the unit, from one stage before the one it is loaded from
+    uint32_t at;      // where unit 0's pieces go in a plane
+
+    // Unit u lies kRows rows (k-contiguous) or kChunks chunks of 8 k (k-major)
+    // after unit u - 1.
+    static constexpr int kRows = NT / 8, kChunks = NT / (2 * R);
+    static_assert(KC ? kRows % 16 == 0 : U == 1 || ((kChunks & (kChunks - 1)) == 0 && kChunks > 0),
+                  "unit 0's address serves all units");
 
     // first k of unit id inside a stage
     static __device__ __forceinline__ int first_k(int id) { return KC ? 4 * (id % 8) : F * (id / R); }
     __device__ __forceinline__ void init(int tid, int64_t ld, int64_t row0, int64_t rows) {
+        const int r0 = KC ? tid / 8 : tid % R, c0 = first_k(tid) / 8;
+        at = (uint32_t)(c0 * R * 16 + (r0 ^ swz(c0)) * 16 + (first_k(tid) & 4) * 2);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int id = tid + u * NT;
@@ -129,7 +142,6 @@ struct X3Loader {
                 const int64_t r = min((int64_t)(id % R), rows - 1 - row0);
                 off[u] = (uint32_t)(((first_k(id) + kBK) * ld + r) * 4);
             }
-            seen[u] = 0;
         }
     }
     // k positions the 8-k group at k is moved down by in a last stage with
@@ -172,37 +184,19 @@ struct X3Loader {
             for (int e = 0; e < F; ++e) v[u][e] = e < drop ? 0.f : v[u][e];
         }
     }
-    __device__ __forceinline__ void store(int u, char *planes, int tid) {
+    __device__ __forceinline__ void store(int u, char *planes) {
         constexpr int CH = R * 16, PL = 4 * CH;
-        const int id = tid + u * NT;
         uint32_t p[3][F / 2];
 #pragma unroll
-        for (int e = 0; e < F; e += 2) split2(v[u][e], v[u][e + 1], p[0][e / 2], p[1][e / 2], p[2][e / 2]);
-#pragma unroll
-        for (int e = 0; e < F / 2; ++e) seen[u] |= p[0][e];
+        for (int e = 0; e < F; e += 2)
+            split2(v[u][e] * kPieceUp, v[u][e + 1] * kPieceUp, p[0][e / 2], p[1][e / 2], p[2][e / 2]);
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            const int r = KC ? id / 8 : id % R, k = first_k(id);
-            char *dst = planes + q * PL + (k / 8) * CH + spread(r, k / 8) * 16 + (k & 4) * 2;
-            *reinterpret_cast<uint2 *>(dst) = make_uint2(p[q][0], p[q][1]);
+            // (k-major: unit 0's chunk is below kChunks, so the chunk bits and
+            // with them the XORs of both combine)
+            char *dst = KC ? planes + at + u * kRows * 16 : planes + (at ^ (swz(u * kChunks) * 16)) + u * kChunks * CH;
+            *reinterpret_cast<uint2 *>(dst + q * PL) = make_uint2(p[q][0], p[q][1]);
         }
-    }
-    // Whether a row of a k-contiguous operand (one of a k-major operand's
-    // columns, over one 8-k group of every stage) has no element of 2^-95 or
-    // more but some below it.
-    __device__ __forceinline__ bool tiny() const {
-        bool t = false;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            uint32_t s = seen[u];
-            if (KC) {  // the eight lanes of a row
-                s |= (uint32_t)__builtin_amdgcn_mov_dpp((int)s, 0xB1, 0xf, 0xf, false);   // quad_perm [1,0,3,2]
-                s |= (uint32_t)__builtin_amdgcn_mov_dpp((int)s, 0x4E, 0xf, 0xf, false);   // quad_perm [2,3,0,1]
-                s |= (uint32_t)__builtin_amdgcn_mov_dpp((int)s, 0x141, 0xf, 0xf, false);  // row_half_mirror
-            }
-            t |= (s & 0x7fff7fffu) != 0 && (s & 0x70007000u) == 0;
-        }
-        return t;
     }
 };
 
@@ -307,8 +301,8 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
     };
 
     bf16x8 af[2][3], bf[2][FN][3];
-    const int fo_a = (lane >> 4) * CHA + (wm0 + spread(lane & 15, lane >> 4)) * 16;
-    const int fo_b = (lane >> 4) * CHB + (wn0 + spread(lane & 15, lane >> 4)) * 16;
+    const int fo_a = (lane >> 4) * CHA + (wm0 + ((lane & 15) ^ swz(lane >> 4))) * 16;
+    const int fo_b = (lane >> 4) * CHB + (wn0 + ((lane & 15) ^ swz(lane >> 4))) * 16;
     auto read_a = [&](int set, int buf, int i) __attribute__((always_inline)) {
         const char *s = ring(buf) + fo_a + i * 256;
 #pragma unroll
@@ -328,30 +322,37 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
         for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     // Product s of the six of row block i, smallest first, into a sum of the
     // stage's own.  Each sum is added to its accumulators while the next row
-    // block's products run (the last block's in the next stage).
-    f32x4 sum[2][FN];
+    // block's products run (the last block's in the next stage): with four or
+    // more column blocks one after another as the next products take their
+    // place, which needs one set of registers, and otherwise from a second set
+    // after the third product, so that no add waits for its MFMA.
+    constexpr int SB = FN >= 4 ? 1 : 2;
+    f32x4 sum[SB][FN];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) sum[1][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto add_sum = [&](int i) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = acc[i][j] + sum[i & 1][j];
-    };
+    for (int j = 0; j < FN; ++j) sum[SB - 1][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto add_sum = [&](int i, int j) __attribute__((always_inline)) { acc[i][j] = acc[i][j] + sum[i % SB][j]; };
     auto step = [&](int i, int s, int aset, int bset) __attribute__((always_inline)) {
         constexpr int P[6] = {2, 1, 0, 1, 0, 0}, Q[6] = {0, 1, 2, 0, 1, 0};
+        const int before = i == 0 ? FM - 1 : i - 1;
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-            sum[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                bf[bset][j][Q[s]], af[aset][P[s]], s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum[i & 1][j], 0, 0, 0);
-        if (s == 2) add_sum(i == 0 ? FM - 1 : i - 1);
+        for (int j = 0; j < FN; ++j) {
+            if (SB == 1 && s == 0) add_sum(before, j);
+            sum[i % SB][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                bf[bset][j][Q[s]], af[aset][P[s]], s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum[i % SB][j], 0, 0, 0);
+        }
+        if (SB == 2 && s == 2) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j) add_sum(before, j);
+        }
     };
 
     before_load(0);
     load(0);
     before_store(0);
 #pragma unroll
-    for (int u = 0; u < UA; ++u) ga.store(u, ring(0), tid);
+    for (int u = 0; u < UA; ++u) ga.store(u, ring(0));
 #pragma unroll
-    for (int u = 0; u < UB; ++u) gb.store(u, ring(0) + G::kABytes, tid);
+    for (int u = 0; u < UB; ++u) gb.store(u, ring(0) + G::kABytes);
     before_load(1);
     load(1);
     wait_lgkm0();
@@ -379,13 +380,15 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
                 for (int s = s0; s < s1; ++s) step(r, s, r & 1, P);
                 constexpr bool isa = u < UA;
                 if constexpr (n > 0 && isa) {
-                    ga.store(u, ring(P ^ 1), tid);
+                    ga.store(u, ring(P ^ 1));
                     ga.load(u, a_next, p.lda);
                 } else if constexpr (n > 0) {
-                    gb.store(u - UA, ring(P ^ 1) + G::kABytes, tid);
+                    gb.store(u - UA, ring(P ^ 1) + G::kABytes);
                     gb.load(u - UA, b_next, p.ldb);
                 }
-                mix<n == 0 ? 0 : (isa ? G::AK : G::BK) ? 1 : 4, n == 0 ? 0 : 24 + 4 * FN / pieces, i == 0 ? 3 : 0, n == 0 ? 0 : 3, (s1 - s0) * FN>();
+                if constexpr (SB == 1 && i == 0) mix<0, 4 * FN, 0, 0, FN>();
+                mix<n == 0 ? 0 : (isa ? G::AK : G::BK) ? 1 : 4, n == 0 ? 0 : 26 + (SB == 2 ? 4 * FN / pieces : 0),
+                    i == 0 ? 3 : 0, n == 0 ? 0 : 3, (s1 - s0 - (SB == 1 && i == 0 ? 1 : 0)) * FN>();
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
@@ -395,23 +398,37 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
         read_a(0, P ^ 1, 0);
 #pragma unroll
         for (int s = 0; s < 6; ++s) step(FM - 1, s, (FM - 1) & 1, P);
-        mix<0, 0, 3 + 3 * FN, 0, 6 * FN>();
+        if constexpr (SB == 1) mix<0, 4 * FN, 0, 0, FN>();
+        mix<0, 0, 3 + 3 * FN, 0, (SB == 1 ? 5 : 6) * FN>();
         __builtin_amdgcn_sched_barrier(0);
+        // The stage's adds stay in the stage: left to itself the compiler
+        // moves them into the blocks after the next branch, past the
+        // scheduling barriers, and every row block's sums stay in registers
+        // until then (256 and 26 to 44 spilled, 1027 us at 4096^3; with this
+        // and the loop in pairs 230 and none).
+#pragma unroll
+        for (int i = 0; i + 1 < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                f32x4 &x = acc[i][j];
+                asm volatile("" : "+v"(x));
+            }
     };
-    for (int t = 0;;) {
+    int t = 0;
+    for (; t + 1 < nk; t += 2) {
         stage(t, std::integral_constant<int, 0>{});
-        if (++t >= nk) break;
-        stage(t, std::integral_constant<int, 1>{});
-        if (++t >= nk) break;
+        stage(t + 1, std::integral_constant<int, 1>{});
     }
-    add_sum(FM - 1);
+    if (t < nk) stage(t, std::integral_constant<int, 0>{});
+#pragma unroll
+    for (int j = 0; j < FN; ++j) add_sum(FM - 1, j);
 
-    // Values the pieces cannot carry: non-finite sums (an infinity splits
-    // into inf and NaN; a leading piece may round up to inf), and rows whose
-    // every element is below 2^-95.  The tile is then computed again on the
-    // f32 matrix instructions, straight from memory.
+    // Values the pieces cannot carry: an infinity splits into inf and NaN, an
+    // element of 2^112 or a sum of 2^96 becomes inf scaled.  Where a sum is
+    // not finite the tile is computed again on the f32 matrix instructions,
+    // straight from memory.
     {
-        int odd = ga.tiny() || gb.tiny();
+        int odd = 0;
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -443,6 +460,11 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
                     for (int j = 0; j < FN; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j], a[i], acc[i][j], 0, 0, 0);
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[i][j] = acc[i][j] * kPieceDown;
         }
     }
 

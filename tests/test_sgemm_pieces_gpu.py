@@ -208,3 +208,44 @@ def test_offset_limits_fall_back(torch_dev):
     assert rc == 0
     s = a.double().abs() @ b.double().abs()
     assert ((out.double() - a.double() @ b.double()).abs() <= (k + 4) * 2.0 ** -24 * s).all()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k", [(70, 130, 96), (300, 200, 40), (33, 64, 2100)])
+def test_small_elements_beside_large_ones(torch_dev, m, n, k, ta, tb):
+    """Elements down to the fp32 subnormals keep their 24 bits next to elements
+    near 1 in the same row: products of theirs are the output where the other
+    operand is zero at the large ones.  Each output within the bar, plus the
+    rounding of a subnormal result."""
+    import torch
+    g = torch.Generator().manual_seed(m + k)
+    for e in (-112, -120, -127, -145):
+        small = torch.randn(m, k, dtype=torch.float64, generator=g) * 2.0 ** e
+        small[:, ::8] = torch.randn(m, (k + 7) // 8, dtype=torch.float64, generator=g)
+        other = torch.randn(k, n, dtype=torch.float64, generator=g) * 2.0 ** 60
+        other[::8, :n // 2] = 0.0
+        for a64, b64 in ((small, other), (other.t(), small.t())):
+            opa, opb = a64.float(), b64.float()
+            a = (opa.t() if ta else opa).contiguous().to(torch_dev)
+            b = (opb.t() if tb else opb).contiguous().to(torch_dev)
+            got = _gh().sgemm(a, b, trans_a=bool(ta), trans_b=bool(tb)).cpu().double()
+            ref, s = opa.double() @ opb.double(), opa.double().abs() @ opb.double().abs()
+            assert ((got - ref).abs() <= (k / 32 + 12) * 2.0 ** -24 * s + 2.0 ** -148).all(), \
+                (e, float(((got - ref).abs() / s).max()))
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_large_sums(torch_dev, ta, tb):
+    """Values and sums up to the largest fp32 ones, finite ones within the f32
+    chain's bound (they leave the range of the pieces)."""
+    import torch
+    m, n, k = 70, 66, 64
+    for ea, eb in ((110, 10), (60, 60), (0, 120), (50, 46)):
+        a, b, opa, opb = _operands(torch, torch_dev, m, n, k, ta, tb, ea)
+        opa.mul_(2.0 ** ea)
+        opb.mul_(2.0 ** eb)
+        out = torch.empty(m, n, device=torch_dev)
+        _sgemm(torch, _gh(), a, b, m, n, k, ta, tb, out)
+        ref, s = opa.double() @ opb.double(), opa.double().abs() @ opb.double().abs()
+        assert out.isfinite().all()
+        assert ((out.double() - ref).abs() <= (k / 2 + 4) * 2.0 ** -24 * s).all()
