@@ -31,10 +31,15 @@
 // 2048 1143 -> 681, not causal 1000 540 -> 314; D = 64 causal 165 -> 103;
 // with weights and a mask B = 4, H = 16, S = 512, D = 64 201 -> 57.
 //
+// V and the probabilities are scaled by 2^16 before they are split (and the
+// sums scaled back), so that small ones keep their 24 bits: a weight of 2^-120
+// can be the output where V is zero at the larger ones.  Q and K need no
+// scale, as a score enters by its absolute size: their lost bits move it by
+// less than 2^-134 2^60 2^20 d (the bounds below), nothing.
+//
 // Inputs beyond the pieces: a workgroup that meets an element of Q, K or V
-// that is not finite or above 2^60 (a tiny piece times it would not be
-// negligible), and a wave whose result is not finite or below 2^-95, redo
-// their queries on f32 MFMAs (set_f32).
+// that is not finite or above 2^60, or a scale above 2^20, and a wave whose
+// result is not finite redo their queries on f32 MFMAs (set_f32).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -120,10 +125,10 @@ struct KvRegs {
             for (int e = 0; e < 4; ++e) x = max_nan(max_nan(fabsf(k[u][e]), fabsf(v[u][e])), x);
         return x;
     }
-    static __device__ __forceinline__ void put(char *at, const float (&x)[4]) {
+    static __device__ __forceinline__ void put(char *at, const float (&x)[4], float up) {
         uint2 p[3];
-        split2(x[0], x[1], p[0].x, p[1].x, p[2].x);
-        split2(x[2], x[3], p[0].y, p[1].y, p[2].y);
+        split2(x[0] * up, x[1] * up, p[0].x, p[1].x, p[2].x);
+        split2(x[2] * up, x[3] * up, p[0].y, p[1].y, p[2].y);
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2 *>(at + q * T::kPlane) = p[q];
     }
@@ -132,13 +137,13 @@ struct KvRegs {
         if (!T::kAll && id >= T::kUnits) return;
         const int key = id / (DP / 4), q = id % (DP / 4), st = q / 8, c = (q % 8) >> 1;
         put(lds + st * (kKeys * 64) + c * (kKeys * 16) + (key & 16) * 16 + ((key & 15) ^ swz(c) ^ st) * 16 + (q & 1) * 8,
-            k[u]);
+            k[u], 1.f);
     }
     __device__ __forceinline__ void store_v(int u, char *lds, int tid) const {
         const int id = tid + u * kThreads;
         if (!T::kAll && id >= T::kUnits) return;
         const int dim = id % DP, kq = id / DP, c = kq & 3;
-        put(lds + c * (DP * 16) + (dim & ~15) * 16 + ((dim & 15) ^ swz(c)) * 16 + (kq >> 2) * 8, v[u]);
+        put(lds + c * (DP * 16) + (dim & ~15) * 16 + ((dim & 15) ^ swz(c)) * 16 + (kq >> 2) * 8, v[u], kPieceUp);
     }
 };
 
@@ -442,7 +447,7 @@ __global__ __launch_bounds__(kThreads, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_
             }
             uint32_t pk[3][4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) split2(pv[2 * e], pv[2 * e + 1], pk[0][e], pk[1][e], pk[2][e]);
+            for (int e = 0; e < 4; ++e) split2(pv[2 * e] * kPieceUp, pv[2 * e + 1] * kPieceUp, pk[0][e], pk[1][e], pk[2][e]);
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 const i32x4 w = {(int)pk[q][0], (int)pk[q][1], (int)pk[q][2], (int)pk[q][3]};
@@ -497,12 +502,12 @@ __global__ __launch_bounds__(kThreads, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float x = fabsf(o[i][b][r]);
-                bad |= !(x <= 3.402823466e38f) || (x != 0.f && x < 2.524354897e-29f);
+                bad |= !(x <= 3.402823466e38f);
             }
         odd |= bad && m[i] != -INFINITY && q < p.sq;
         l[i] = inv_l;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) o[i][b] *= inv_l;
+        for (int b = 0; b < NB; ++b) o[i][b] = o[i][b] * kPieceDown * inv_l;
     }
     odd = __any(odd);
     if (live && !odd) {

@@ -230,3 +230,43 @@ def test_nan_scores_many_slices(torch_dev):
         for x in r if weights else (r,):
             assert x[7, 9].isnan().all()
             assert x[7, 8].isfinite().all() and x[7, 10].isfinite().all()
+
+
+@pytest.mark.parametrize("d", [4, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_small_weights_and_values(torch_dev, causal, d):
+    """A weight of 2^-124 keeps fp32 precision where V is zero at the larger
+    ones, and V down to the subnormals keeps its bits.  Scores are exact here
+    (one product of small integers each), so a weight is within |s| 2^-23 (the
+    exponent's product) + 2^-19 (the rounded exponent of up to 2^7, times
+    ln 2) + 8 2^-24, and the output 8 2^-24 more."""
+    import torch
+    gh = _gh()
+    s = 40
+    q, k = torch.zeros(1, 2, s, d, device=torch_dev), torch.zeros(1, 2, s, d, device=torch_dev)
+    q[..., 0] = 2.0
+    k[..., 0] = -86.0
+    k[:, :, 0, 0] = 0.0
+    scale = 0.5
+    g = torch.Generator(device=torch_dev).manual_seed(d)
+    for e in (50, 0, -20):
+        v = torch.randn(1, 2, s, d, device=torch_dev, generator=g) * 2.0 ** e
+        v[:, :, 0] = 0.0
+        got = gh.sdpa(q, k, v, scale=scale, causal=causal)
+        x = (q.double() @ k.double().transpose(-1, -2).contiguous()) * scale
+        if causal:
+            x = x.masked_fill(~torch.ones(s, s, dtype=torch.bool, device=torch_dev).tril(), -math.inf)
+        w = torch.softmax(x, -1)
+        ref, bar = w @ v.double(), w @ v.double().abs()
+        # (fp32 weights and outputs below 2^-126 round to 2^-149)
+        assert ((got.double() - ref).abs() <= bar * (86 * 2.0 ** -23 + 2.0 ** -19 + 16 * 2.0 ** -24) + s * 2.0 ** -148).all(), \
+            (e, float(((got.double() - ref).abs() / bar.clamp_min(1e-300)).max()))
+    # subnormal values under ordinary weights
+    q, k = (torch.randn(1, 2, s, d, device=torch_dev, generator=g) for _ in range(2))
+    for e in (-118, -130, -140):
+        v64 = torch.randn(1, 2, s, d, device=torch_dev, generator=g).double() * 2.0 ** e
+        v = v64.float()
+        got = gh.sdpa(q, k, v, causal=causal)
+        keep = _kept(torch, 1, 2, s, s, causal, None, torch_dev)
+        ref, _, bar, _ = _reference(torch, q, k, v, keep, 1.0 / math.sqrt(d))
+        assert ((got.double() - ref).abs() <= bar - s * 2.0 ** -126 + 2.0 ** -148).all(), e
