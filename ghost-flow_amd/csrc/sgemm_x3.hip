@@ -573,14 +573,6 @@ void launch_layouts(const SgemmDesc &d, const X3Params &p, dim3 grid, hipStream_
 
 }  // namespace
 
-// Whether this kernel takes the product.  K >= 32: below that the fp32 chain
-// is short enough for its rounding to be smaller than the pieces'.  The
-// operand offsets inside a tile are 32-bit.
-bool sgemm_x3_fits(const SgemmDesc &d) {
-    constexpr int64_t kMaxLd = 1 << 21;
-    return d.k >= 32 && d.k <= (int64_t)1 << 30 && d.m >= 1 && d.n >= 1 && d.lda <= kMaxLd && d.ldb <= kMaxLd;
-}
-
 namespace {
 
 struct X3Plan {
@@ -601,12 +593,19 @@ struct X3Plan {
 struct X3Tile {
     int bm, bn, per_cu;
     double alone, full, ends;
+    int threads() const { return bm == 32 ? 256 : 512; }
+    int64_t tiles(const SgemmDesc &d, int64_t count) const {
+        return ((d.m + bm - 1) / bm) * ((d.n + bn - 1) / bn) * count;
+    }
 };
 constexpr X3Tile kTiles[] = {{256, 128, 1, 1.75, 2.20, 4.5},
                              {128, 128, 1, 1.00, 1.32, 2.2},
                              {128, 64, 2, 0.64, 0.71, 1.1},
                              {64, 64, 3, 0.48, 0.44, 0.5},
                              {32, 64, 4, 0.44, 0.30, 0.3}};
+
+// Work items of a launch: 32 bits.
+bool x3_grid_fits(const X3Tile &t, int64_t workgroups) { return workgroups * t.threads() < (int64_t)1 << 32; }
 
 // The tile and K split with the shortest estimated time for `count` products
 // of one shape: workgroups in rounds of per_cu on every CU.  K slices (unless
@@ -618,7 +617,8 @@ X3Plan plan_x3(const SgemmDesc &d, int64_t count, bool split) {
     double least = 1e30;
     for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
         const X3Tile &t = kTiles[i];
-        const int64_t tiles = ((d.m + t.bm - 1) / t.bm) * ((d.n + t.bn - 1) / t.bn) * count;
+        const int64_t tiles = t.tiles(d, count);
+        if (!x3_grid_fits(t, tiles)) continue;
         const int64_t round = (int64_t)t.per_cu * 256;
         for (int sl = 1; sl <= (split ? 16 : 1); ++sl) {
             const double one = (double)t.bm * t.bn * 4, part = (double)sl * (double)tiles * one;
@@ -636,6 +636,12 @@ X3Plan plan_x3(const SgemmDesc &d, int64_t count, bool split) {
         }
     }
     return best;
+}
+
+bool x3_takes(const SgemmDesc &d, int64_t count) {
+    constexpr int64_t kMaxLd = 1 << 21;
+    return d.k >= 32 && d.k <= (int64_t)1 << 30 && d.m >= 1 && d.n >= 1 && d.lda <= kMaxLd && d.ldb <= kMaxLd &&
+           x3_grid_fits(kTiles[0], kTiles[0].tiles(d, count));
 }
 
 // d[0] gives the shape and layout of all products.
@@ -674,6 +680,13 @@ int launch_products(const SgemmDesc *d, X3Params &p, hipStream_t s) {
 
 }  // namespace
 
+// Whether this kernel takes the product.  K >= 32: below that the fp32 chain
+// is short enough for its rounding to be smaller than the pieces'.  The
+// operand offsets inside a tile are 32-bit, and so is the number of threads of
+// the launch: from 2^29 rows on the smaller tiles drop out (128 x 64 has four
+// threads a row), at 2^31 the largest.
+bool sgemm_x3_fits(const SgemmDesc &d) { return x3_takes(d, std::max<int64_t>(d.batch, 1)); }
+
 int launch_sgemm_x3(const SgemmDesc &d, hipStream_t s) {
     X3Params p{};
     p.a[0] = d.a;
@@ -696,7 +709,7 @@ bool sgemm_x3_group_fits(const SgemmDesc *d, int count) {
     if (count < 1 || count > kNtMaxGroups) return false;
     for (int g = 0; g < count; ++g) {
         const SgemmDesc &e = d[g];
-        if (!sgemm_x3_fits(e) || e.batch > 1 || e.batch_a > 1 || e.batch_b > 1 || e.trans_a != d[0].trans_a ||
+        if (!x3_takes(e, count) || e.batch > 1 || e.batch_a > 1 || e.batch_b > 1 || e.trans_a != d[0].trans_a ||
             e.trans_b != d[0].trans_b || e.m != d[0].m || e.n != d[0].n || e.k != d[0].k || e.lda != d[0].lda ||
             e.ldb != d[0].ldb || e.alpha != d[0].alpha || e.beta != d[0].beta)
             return false;
@@ -720,3 +733,29 @@ int launch_sgemm_x3_group(const SgemmDesc *d, int count, hipStream_t s) {
 }
 
 }  // namespace gfh
+
+// What the plan gives an [m, k] x [k, n] product: out = {tile rows, tile
+// columns, K slices, threads of the launch}; returns 0 where the kernel does
+// not take it.  Not part of the API: it lets the tests say which tile a shape
+// runs on, without a GPU.
+extern "C" __attribute__((visibility("default"))) int gfh_internal_sgemm_x3_plan(int trans_a, int trans_b, int64_t m,
+                                                                                 int64_t n, int64_t k, int64_t batch,
+                                                                                 int64_t *out) {
+    gfh::SgemmDesc d;
+    d.trans_a = trans_a != 0;
+    d.trans_b = trans_b != 0;
+    d.m = m;
+    d.n = n;
+    d.k = k;
+    d.lda = trans_a ? m : k;
+    d.ldb = trans_b ? k : n;
+    d.batch = batch;
+    if (!gfh::sgemm_x3_fits(d)) return 0;
+    const gfh::X3Plan plan = gfh::plan_x3(d, batch, batch == 1);
+    const gfh::X3Tile &t = gfh::kTiles[plan.tile];
+    out[0] = t.bm;
+    out[1] = t.bn;
+    out[2] = plan.slices;
+    out[3] = t.tiles(d, batch) * plan.slices * t.threads();
+    return 1;
+}

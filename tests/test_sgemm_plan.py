@@ -1,0 +1,32 @@
+"""The tile and K split that the fp32 GEMM's plan picks (sgemm_x3.hip), on the
+CPU: it is host code."""
+import ctypes as C
+
+import pytest
+
+
+def plan(m, n, k, ta=0, tb=0, batch=1):
+    """(tile rows, tile columns, K slices, threads), or None where another
+    kernel takes the product."""
+    import ghostflow_hip
+    f = C.CDLL(ghostflow_hip.lib()._name).gfh_internal_sgemm_x3_plan
+    f.argtypes = [C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.POINTER(C.c_int64)]
+    out = (C.c_int64 * 4)()
+    return tuple(out) if f(ta, tb, m, n, k, batch, out) else None
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(1 << 29, 1, 32, 1), (1 << 30, 1, 32, 1), (1 << 30, 40, 32, 1),
+                                         ((1 << 31) - 1000, 8, 32, 1), (1, 1 << 21, 32, 500), (200, 1 << 21, 32, 500),
+                                         (1 << 14, 1, 32, 65535)])
+def test_launches_stay_within_32_bits(m, n, k, batch):
+    """A grid of 2^32 threads is refused by the runtime: tiles that would need
+    one are not picked."""
+    bm, bn, slices, threads = plan(m, n, k, batch=batch)
+    assert threads < 1 << 32
+
+
+def test_beyond_every_tile():
+    """Where the largest tile's grid is too large the product is left to the
+    f32 tile kernel."""
+    assert plan((1 << 31) - 1, 8, 32) is None and plan(1, 1 << 21, 32, batch=512) is None
+    assert plan(1 << 30, 128, 32) is not None and plan(1 << 30, 129, 32) is None
