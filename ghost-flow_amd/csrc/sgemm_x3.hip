@@ -52,6 +52,7 @@
 //    sums of 2^96 and more are computed again on the f32 instructions
 //    (sgemm_x3_kernel's end).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -81,9 +82,10 @@ struct X3Geo {
     static constexpr int kStage = kABytes + kBBytes;
     static constexpr int kLds = 2 * kStage;
     static_assert(kLds <= 160 * 1024, "LDS per workgroup");
-    // workgroups per CU that the LDS leaves room for
+    // workgroups per CU that the LDS leaves room for, and the register bound
+    // that lets all of them in
     static constexpr int kPerCu = (160 * 1024) / kLds;
-    static constexpr int kWavesPerSimd = std::max(1, std::min(4, kPerCu * NT / 256));
+    static constexpr int kWavesPerSimd = std::max(1, kPerCu * NT / 256);
 };
 
 struct X3Params {
@@ -555,31 +557,6 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
     }
 }
 
-template <int BM, int BN, int NWM, int NWN>
-void launch_layouts(const SgemmDesc &d, const X3Params &p, dim3 grid, hipStream_t s) {
-    const dim3 block(64 * NWM * NWN);
-    if (d.trans_a) {
-        if (d.trans_b)
-            hipLaunchKernelGGL((sgemm_x3_kernel<X3Geo<BM, BN, NWM, NWN, false, true>>), grid, block, 0, s, p);
-        else
-            hipLaunchKernelGGL((sgemm_x3_kernel<X3Geo<BM, BN, NWM, NWN, false, false>>), grid, block, 0, s, p);
-    } else {
-        if (d.trans_b)
-            hipLaunchKernelGGL((sgemm_x3_kernel<X3Geo<BM, BN, NWM, NWN, true, true>>), grid, block, 0, s, p);
-        else
-            hipLaunchKernelGGL((sgemm_x3_kernel<X3Geo<BM, BN, NWM, NWN, true, false>>), grid, block, 0, s, p);
-    }
-}
-
-}  // namespace
-
-namespace {
-
-struct X3Plan {
-    int tile;  // index into kTiles
-    int slices;
-};
-
 // Tiles and what they take (us): a stage of 32 k where a workgroup has its CU
 // to itself, the same per workgroup of a filled GPU (less where several share
 // a CU and hide each other's latency; more at 256x128 and 128x128, one per CU,
@@ -593,7 +570,7 @@ struct X3Plan {
 struct X3Tile {
     int bm, bn, per_cu;
     double alone, full, ends;
-    int threads() const { return bm == 32 ? 256 : 512; }
+    constexpr int threads() const { return bm == 32 ? 256 : 512; }
     int64_t tiles(const SgemmDesc &d, int64_t count) const {
         return ((d.m + bm - 1) / bm) * ((d.n + bn - 1) / bn) * count;
     }
@@ -604,6 +581,30 @@ constexpr X3Tile kTiles[] = {{256, 128, 1, 1.75, 2.20, 4.5},
                              {64, 64, 3, 0.48, 0.44, 0.5},
                              {32, 64, 4, 0.44, 0.30, 0.3}};
 
+// Tile I of the table on an NWM x NWN wave grid, in the layout of d.
+template <int I, int NWM, int NWN>
+void launch_tile(const SgemmDesc &d, const X3Params &p, dim3 grid, hipStream_t s) {
+    constexpr int BM = kTiles[I].bm, BN = kTiles[I].bn;
+    static_assert(X3Geo<BM, BN, NWM, NWN, true, true>::kPerCu == kTiles[I].per_cu &&
+                      64 * NWM * NWN == kTiles[I].threads(),
+                  "the plan's figures are the kernel's");
+    auto go = [&](auto ak, auto bk) {
+        hipLaunchKernelGGL((sgemm_x3_kernel<X3Geo<BM, BN, NWM, NWN, decltype(ak)::value, decltype(bk)::value>>), grid,
+                           dim3(64 * NWM * NWN), 0, s, p);
+    };
+    using Y = std::true_type;
+    using N = std::false_type;
+    if (d.trans_a)
+        d.trans_b ? go(N{}, Y{}) : go(N{}, N{});
+    else
+        d.trans_b ? go(Y{}, Y{}) : go(Y{}, N{});
+}
+
+struct X3Plan {
+    int tile;  // index into kTiles
+    int slices;
+};
+
 // Work items of a launch: 32 bits.
 bool x3_grid_fits(const X3Tile &t, int64_t workgroups) { return workgroups * t.threads() < (int64_t)1 << 32; }
 
@@ -612,14 +613,14 @@ bool x3_grid_fits(const X3Tile &t, int64_t workgroups) { return workgroups * t.t
 // batched) add the partial tiles' stores, at 6 TB/s, and the last arriver's
 // reads of a tile's partials, which one workgroup takes in at 100 GB/s.
 X3Plan plan_x3(const SgemmDesc &d, int64_t count, bool split) {
-    const int64_t stages = (d.k + kBK - 1) / kBK;
+    const int64_t stages = (d.k + kBK - 1) / kBK, cus = device_cu_count();
     X3Plan best{0, 1};
     double least = 1e30;
     for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
         const X3Tile &t = kTiles[i];
         const int64_t tiles = t.tiles(d, count);
         if (!x3_grid_fits(t, tiles)) continue;
-        const int64_t round = (int64_t)t.per_cu * 256;
+        const int64_t round = t.per_cu * cus;
         for (int sl = 1; sl <= (split ? 16 : 1); ++sl) {
             const double one = (double)t.bm * t.bn * 4, part = (double)sl * (double)tiles * one;
             if (sl > 1 && (stages / sl < 4 || part > 64e6)) break;
@@ -627,7 +628,7 @@ X3Plan plan_x3(const SgemmDesc &d, int64_t count, bool split) {
             const double st = (double)((stages + sl - 1) / sl);
             auto shared = [&](double n) { return std::max(st * t.alone, n * st * t.full) + n * t.ends; };
             double us = (double)(tasks / round) * shared(t.per_cu);
-            if (rem) us += rem <= 192 ? st * t.alone + t.ends : shared((double)((rem + 255) / 256));
+            if (rem) us += 4 * rem <= 3 * cus ? st * t.alone + t.ends : shared((double)((rem + cus - 1) / cus));
             if (sl > 1) us += 2.5 + part / 6e6 + sl * one / 1e5;
             if (us < least) {
                 least = us;
@@ -669,11 +670,11 @@ int launch_products(const SgemmDesc *d, X3Params &p, hipStream_t s) {
     }
     const dim3 grid((unsigned)(nblk * p.slices));
     switch (plan.tile) {
-        case 0: launch_layouts<256, 128, 4, 2>(*d, p, grid, s); break;
-        case 1: launch_layouts<128, 128, 2, 4>(*d, p, grid, s); break;
-        case 2: launch_layouts<128, 64, 4, 2>(*d, p, grid, s); break;
-        case 3: launch_layouts<64, 64, 2, 4>(*d, p, grid, s); break;
-        default: launch_layouts<32, 64, 1, 4>(*d, p, grid, s); break;
+        case 0: launch_tile<0, 4, 2>(*d, p, grid, s); break;
+        case 1: launch_tile<1, 2, 4>(*d, p, grid, s); break;
+        case 2: launch_tile<2, 4, 2>(*d, p, grid, s); break;
+        case 3: launch_tile<3, 2, 4>(*d, p, grid, s); break;
+        default: launch_tile<4, 1, 4>(*d, p, grid, s); break;
     }
     return check_launch("sgemm (bf16 pieces)");
 }
