@@ -11,6 +11,8 @@ import ctypes as C
 
 import pytest
 
+from test_sgemm_plan import plan
+
 pytestmark = pytest.mark.gpu
 
 
@@ -108,6 +110,34 @@ def test_batches_modulo(torch_dev, m, n, k, ba, bb, batch):
         for i in range(batch):
             x, y = a[i % ba], b[i % bb]
             _check(torch, out[i], x.t() if ta else x, y.t() if tb else y, k)
+
+
+@pytest.mark.parametrize("m,n,k,ba,bb,batch", [(32, 345, 1742, 2, 2, 2), (411, 140, 2100, 3, 1, 6), (40, 100, 4100, 4, 2, 4),
+                                               (500, 64, 4096, 2, 2, 2)])
+def test_batches_split_k(torch_dev, m, n, k, ba, bb, batch):
+    """Batches whose K is split: every slice's own partials and counters, with
+    alpha, beta and a bias, the same bits from call to call."""
+    import torch
+    for ta, tb in ((0, 0), (0, 1), (1, 0), (1, 1)):
+        assert plan(m, n, k, ta, tb, batch)[2] > 1
+        a = torch.randn((ba,) + ((k, m) if ta else (m, k)), device=torch_dev)
+        b = torch.randn((bb,) + ((n, k) if tb else (k, n)), device=torch_dev)
+        bias, c0 = torch.randn(n, device=torch_dev), torch.randn(batch, m, n, device=torch_dev)
+
+        def call(out, alpha, beta, bias):
+            rc = _gh().lib().gfh_sgemm_strided_batched(
+                ta, tb, m, n, k, alpha, a.data_ptr(), a.shape[2], m * k, ba, b.data_ptr(), b.shape[2], n * k, bb, beta,
+                out.data_ptr(), n, m * n, batch, bias, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0
+            return out
+
+        plain = call(torch.empty_like(c0), 1.0, 0.0, None)
+        for i in range(batch):
+            x, y = a[i % ba], b[i % bb]
+            _check(torch, plain[i], x.t() if ta else x, y.t() if tb else y, k)
+        want = (plain * 0.7 + c0 * -1.3) + bias
+        for _ in range(3):
+            assert torch.equal(call(c0.clone(), 0.7, -1.3, bias.data_ptr()), want)
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
