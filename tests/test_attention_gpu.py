@@ -152,9 +152,8 @@ def test_config5_s2048_sampled_slices(torch_dev):
 
 
 def test_long_sequence_s4096(torch_dev):
-    """S=4096, d=128, causal, 2 (b,h) slices: 128 key tiles per heavy query
-    set and 64 workgroups per slice in the balanced-set kernel, against the
-    oracle; the last query row is the mean-weighted sum over all 4096 keys."""
+    """S=4096, d=128, causal, 2 (b,h) slices: 128 key tiles for the last
+    queries, 32 workgroups per slice, against the oracle; the last query row is the mean-weighted sum over all 4096 keys."""
     gh, O = _gh(), _O()
     shape = (1, 2, 4096, 128)
     q = gh.normal(shape, seed=3, tensor_id=0)

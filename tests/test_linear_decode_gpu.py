@@ -1,7 +1,7 @@
 """Linear::forward at decode sizes (x [m <= 64, k] . W^T, W [out, in]) on the
-GPU: gfh_sgemm sends these NT calls to the row-dot GEMV kernel (m <= 4) or
-to the skinny f32-MFMA kernel (4 < m <= 64).  Against
-the oracle's Linear::forward / matmul (ghostflow-nn/src/linear.rs:56-69,
+GPU: gfh_sgemm sends these NT calls to the row-dot GEMV kernel (m <= 4), to
+the skinny f32-MFMA kernel (4 < m <= 32) or to the tiles on bf16 pieces.
+Against the oracle's Linear::forward / matmul (ghostflow-nn/src/linear.rs:56-69,
 ghostflow-core/src/ops/matmul.rs:91-170).  Bars: bit-exact on
 integer-valued inputs (every partial sum exact in any order), otherwise the
 north-star GEMM bound."""

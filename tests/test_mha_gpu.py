@@ -95,8 +95,8 @@ def test_causal_flag_equals_lower_triangular_mask(torch_dev, sq, p):
     vc[:, :p] = to_dev(pv, torch_dev)
     dx = to_dev(x, torch_dev)
     dm = to_dev(mask, torch_dev)
-    # with the weights output (the 32-query kernel) and without it (the
-    # balanced-set kernel): the flag and the mask agree bit for bit on each
+    # with the weights output and without it: the flag and the mask agree bit
+    # for bit on each
     out, w = gh.mha_forward_cached(dx, dx, dx, *dev, h, kc, vc, p, causal=True, want_weights=True)
     assert_rel(to_np(out), ref[0])
     assert_rel(to_np(w), ref[1])

@@ -43,10 +43,10 @@ def test_reference_known_answers(torch_dev):
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_integer_inputs_bit_exact(torch_dev, m, k, n, ta, tb):
     """|a|,|b| <= 8 integers: every partial sum < 2^24 is exact, so the GPU
-    must equal the oracle bit for bit whatever the summation order.  The
-    shapes cover all three tilings (64x64 below 128 tiles of 128x128,
-    128x64 up to 512 of them, 128x128 beyond) with ragged edges, and long K
-    on few tiles (300 x 4100 x 200)."""
+    must equal the oracle bit for bit whatever the summation order.  K below
+    32 runs on the f32 tile kernel, the rest on bf16 pieces (whose low two
+    are zero for such integers) with ragged edges, and long K on few tiles
+    (300 x 4100 x 200)."""
     gh, O = _gh(), _oracle()
     rng = np.random.default_rng(m * 1000003 + k * 1009 + n)
     a = rng.integers(-8, 9, size=(m, k)).astype(np.float32)
@@ -109,10 +109,10 @@ def test_beta_zero_ignores_nan_output(torch_dev):
 @pytest.mark.parametrize("m,n,k,tb", [(4096, 4096, 32, True), (2048, 2048, 32, False), (2100, 2000, 32, True),
                                       (512, 512, 64, False), (16, 4096, 256, True), (2, 1000, 512, True)])
 def test_beta_zero_ignores_nan_output_every_path(torch_dev, m, n, k, tb):
-    """The same contract on every kernel gfh_sgemm routes to: 256 x 256,
-    128 x 128 with 3 and 2 ring stages, 64 x 64 (direct-to-LDS tiles), the
-    skinny MFMA kernel (16 rows) and the row-dot GEMV (2 rows), with a bias;
-    integer data, so the result is exact."""
+    """The same contract on every kernel gfh_sgemm routes to: the tiles on
+    bf16 pieces (256 x 128 to 32 x 64), the skinny MFMA kernel (16 rows) and
+    the row-dot GEMV (2 rows), with a bias; integer data, so the result is
+    exact."""
     import torch
     gh, O = _gh(), _oracle()
     rng = np.random.default_rng(m + n + k)
@@ -198,15 +198,14 @@ def test_k_zero_gives_bias(torch_dev):
 @pytest.mark.parametrize("tb", [True, False])
 @pytest.mark.parametrize("ta", [False, True])
 def test_big_tiles_integer_exact(torch_dev, m, n, k, tb, ta):
-    """The four layouts with K % 32 == 0 (B as Linear's [n, k] weight or
-    Tensor::matmul's [k, n]; A as [m, k] or, transposed as matmul_backward's
-    a^T, [k, m]) take the direct-to-LDS kernel: 256 x 256 tiles (the first
-    two: K >= 256), 128 x 128 tiles with 2 stages (4352 x 3900, 2100 x 2000)
-    or a 3-deep ring (one round of tiles: 2048^2, 1024 x 4096), and 64 x 64
-    tiles on 2 x 2 waves (the last three) -- ragged m and n inside the last
-    tiles, alpha, beta and bias, on integer data (exact in any summation
-    order).  The reference is the oracle's Linear::forward, or for the
-    largest products the same sums in float64, which are exact here."""
+    """The four layouts (B as Linear's [n, k] weight or Tensor::matmul's [k,
+    n]; A as [m, k] or, transposed as matmul_backward's a^T, [k, m]) with
+    whole K stages: 256 x 128 tiles (the first two) down to 64 x 64 --
+    ragged m and n inside the last tiles, alpha, beta and bias, on integer
+    data (exact in any summation order; test_sgemm_pieces_gpu.py has random
+    data, which fills all three pieces).  The reference is the oracle's
+    Linear::forward, or for the largest products the same sums in float64,
+    which are exact here."""
     gh, O = _gh(), _oracle()
     rng = np.random.default_rng(m + n + k)
     a = rng.integers(-4, 5, size=(m, k)).astype(np.float32)
@@ -230,13 +229,11 @@ def test_big_tiles_integer_exact(torch_dev, m, n, k, tb, ta):
                                    (24, 11008, 2048)])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 def test_big_tiles_split_k_integer_exact(torch_dev, m, n, k, ta, tb):
-    """Launches that split K over the CUs (2-8 slices whose partial tiles the
-    last slice to arrive sums in slice order): fewer than 256 tiles of 64 x
-    64 (32 x 64 up to 32 rows: 17, 24 and 32 rows here), 128 x 128 tiles
-    where those fill more CUs (768 x 760), and 128 x 128 tiles two per CU
-    that fill a partial round (384 x 11000: 258 tiles in 4 slices); ragged m
-    and n, alpha, beta and bias, on integer data (exact in any order); the
-    same call twice, so the arrival counters are back at zero."""
+    """Launches that split K over the CUs, nearly all of these (slices whose
+    partial tiles the last one to arrive sums in slice order; NT with at most
+    32 rows runs on the skinny kernel, split too); ragged m and n, alpha,
+    beta and bias, on integer data (exact in any order); the same call twice,
+    so the arrival counters are back at zero."""
     gh = _gh()
     rng = np.random.default_rng(m + 3 * n + k + 5 * ta + tb)
     if ta and m % 4:
@@ -289,20 +286,18 @@ def _strided_batched(torch_dev, ta, tb, a, b, batch_a, batch_b, batch, m, n, k, 
 
 
 @pytest.mark.parametrize("batch,batch_a,batch_b,m,n,k", [
-    (4, 4, 1, 2048, 2048, 256),   # 256 x 256 tiles, B shared by every slice
-    (16, 16, 16, 512, 512, 128),  # 128 x 128 tiles, one round (3-deep ring), the SDPA score shape
-    (32, 32, 32, 512, 512, 96),   # 128 x 128 tiles, 2 stages
-    (6, 3, 6, 256, 320, 96),      # 64 x 64 tiles, A slices taken modulo 3
-    (6, 6, 3, 300, 260, 64),      # 64 x 64 tiles, B slices modulo 3, ragged edges
+    (4, 4, 1, 2048, 2048, 256),   # the largest tiles, B shared by every slice
+    (16, 16, 16, 512, 512, 128),  # the SDPA score shape
+    (32, 32, 32, 512, 512, 96),
+    (6, 3, 6, 256, 320, 96),      # A slices taken modulo 3
+    (6, 6, 3, 300, 260, 64),      # B slices modulo 3, ragged edges
 ])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
 def test_big_tiles_batched_modulo(torch_dev, batch, batch_a, batch_b, m, n, k, ta, tb):
     """Strided-batched products: slice z multiplies A slice z % batch_a by B
     slice z % batch_b (batched_matmul's modulo indexing, matmul.rs:148-149),
     on integer data (exact in any order), plain and with alpha, beta and
-    bias.  With A as [m, k] they run on the
-    direct-to-LDS kernel, the batch as its grid's y dimension; a transposed
-    A takes the general tile kernel."""
+    bias."""
     rng = np.random.default_rng(batch * 7 + m + n + k + 3 * ta + tb)
     a = rng.integers(-4, 5, size=(batch_a, m, k)).astype(np.float32)
     b = rng.integers(-4, 5, size=(batch_b, k, n)).astype(np.float32)
@@ -320,6 +315,24 @@ def test_big_tiles_batched_modulo(torch_dev, batch, batch_a, batch_b, m, n, k, t
     for z in range(batch):
         prod = (a[z % batch_a].astype(np.float64) @ b[z % batch_b].astype(np.float64)).astype(np.float32)
         np.testing.assert_array_equal(got[z], (2.0 * prod - c0[z] + bias).astype(np.float32), err_msg=f"slice {z}")
+
+
+@pytest.mark.parametrize("m,n,k", [(4200, 3000, 31), (4100, 2300, 16), (1500, 1600, 17), (1500, 1600, 28),
+                                   (200, 130, 30)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_short_k_tiles(torch_dev, m, n, k, ta, tb):
+    """K below 32 stays on the f32 tile kernel: its three tilings (128 x 128
+    from 512 tiles of that size on, 128 x 64 from 128, 64 x 64), with and
+    without 16-byte loads, on random data.  Each output within k + 4 roundings
+    of the sum of the magnitudes."""
+    import torch
+    gh = _gh()
+    g = torch.Generator(device=torch_dev).manual_seed(m + n + k)
+    a = torch.randn((k, m) if ta else (m, k), device=torch_dev, generator=g)
+    b = torch.randn((n, k) if tb else (k, n), device=torch_dev, generator=g)
+    got = gh.sgemm(a, b, trans_a=bool(ta), trans_b=bool(tb)).double()
+    a64, b64 = (a.t() if ta else a).double(), (b.t() if tb else b).double()
+    assert ((got - a64 @ b64).abs() <= (k + 4) * 2.0 ** -24 * (a64.abs() @ b64.abs())).all()
 
 
 @pytest.mark.parametrize("m", [1, 3, 8, 13, 16])
@@ -341,9 +354,8 @@ def test_matmul_decode_rows(torch_dev, m):
 
 @pytest.mark.parametrize("n", [2048, 4096])
 def test_big_tiles_nn_random(torch_dev, n):
-    """NN at n^3 on N(0,1) data (the sweep's shapes: 128 x 128 tiles at 2048,
-    256 x 256 at 4096) against the oracle on sampled rows, within the GEMM
-    bound."""
+    """NN at n^3 on N(0,1) data (256 x 128 tiles) against the oracle on
+    sampled rows, within the GEMM bound."""
     gh, O = _gh(), _oracle()
     rng = np.random.default_rng(8)
     a = rng.standard_normal((n, n)).astype(np.float32)
@@ -356,8 +368,8 @@ def test_big_tiles_nn_random(torch_dev, n):
 
 @pytest.mark.parametrize("m,n", [(4096, 4096), (1000, 900)])
 def test_nt_big_tiles_strided(torch_dev, m, n):
-    """lda > k and ldc > n on the 256 x 256 and the 64 x 64 kernels; bytes
-    between rows of C stay untouched."""
+    """lda > k and ldc > n on a large and a small tile; bytes between rows of C
+    stay untouched."""
     import torch
     gh, O = _gh(), _oracle()
     rng = np.random.default_rng(31)

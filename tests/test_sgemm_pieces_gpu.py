@@ -55,14 +55,17 @@ def _check(torch, got, opa, opb, k):
         float(((got.double() - ref).abs() / s).max())
 
 
-# every tile size is reached: 32-row tiles (m <= 32), 64 x 64, 128 x 64,
-# 128 x 128 and 256 x 128, with remainders of rows, columns and K
+# remainders of rows, columns and K on the 32 x 64, 64 x 64, 128 x 64 and 128 x
+# 128 tiles, and on the 256 x 128 one, whole and with K split
+# (test_sgemm_plan.py checks which tiles these are)
 SHAPES = [(17, 70, 33), (32, 640, 1000), (40, 100, 63), (65, 129, 97), (64, 64, 32), (130, 257, 64), (500, 500, 95),
           (1000, 700, 45), (700, 1500, 401), (2000, 1100, 129), (4100, 2050, 70), (96, 512, 4099)]
+LARGE = [(4090, 4090, 1000), (4000, 4000, 401), (5000, 3000, 129), (2050, 2050, 525), (900, 1000, 8201),
+         (2000, 2060, 4099)]
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("m,n,k", SHAPES + LARGE)
 def test_edges_and_layouts(torch_dev, m, n, k, ta, tb):
     import torch
     gh = _gh()

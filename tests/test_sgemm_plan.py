@@ -30,3 +30,18 @@ def test_beyond_every_tile():
     f32 tile kernel."""
     assert plan((1 << 31) - 1, 8, 32) is None and plan(1, 1 << 21, 32, batch=512) is None
     assert plan(1 << 30, 128, 32) is not None and plan(1 << 30, 129, 32) is None
+
+
+def test_shapes_of_the_gpu_tests_reach_every_tile():
+    """The kernel's tests name shapes, not tiles: a refit of the plan must not
+    leave a tile, or its split form, without its remainders."""
+    from test_sgemm_pieces_gpu import LARGE, SHAPES
+    tiles = {(32, 64), (64, 64), (128, 64), (128, 128), (256, 128)}
+    plans = {s: plan(*s) for s in SHAPES + LARGE}
+    ragged = {s: p for s, p in plans.items() if s[0] % p[0] and s[1] % p[1] and s[2] % 32}
+    assert {p[:2] for p in ragged.values()} == tiles
+    assert all(plans[s][:2] == (256, 128) for s in LARGE)
+    assert {p[2] > 1 for s, p in ragged.items() if s in LARGE} == {False, True}
+    # the four layouts run the same tile
+    for s, p in plans.items():
+        assert {plan(*s, ta, tb) for ta in (0, 1) for tb in (0, 1)} == {p}
