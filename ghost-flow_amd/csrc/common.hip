@@ -164,6 +164,9 @@ struct ScratchBlock {
     void *p = nullptr;
     size_t bytes = 0;
     bool busy = false;
+    uint64_t last = 0;          // g_block_calls when it was last taken
+    hipEvent_t done = nullptr;  // after its last use, where `recorded`
+    bool recorded = false;
 };
 // Needs above kBlockMax, and blocks past kBlockTotal over all streams, are
 // allocated and freed per call: there the kernels outlast the ~17 us of host
@@ -171,9 +174,41 @@ struct ScratchBlock {
 // 4096 x 11008, 21 us of kernels: 25 to 30 us per call of the C entry with
 // them, 21 without).
 constexpr size_t kBlockMax = (size_t)64 << 20, kBlockTotal = (size_t)256 << 20;
+// Nothing tells when a stream is destroyed, so a block goes to another stream
+// once kBlockIdle calls have passed it by and the total leaves no other room.
+// The new owner waits for an event that the old stream recorded after its last
+// use; blocks record one from half the total on, so that programs with a few
+// streams do not pay for it.
+constexpr uint64_t kBlockIdle = 256;
 std::mutex g_block_mu;
 std::map<std::pair<int, hipStream_t>, ScratchBlock> g_blocks;
 size_t g_block_bytes = 0;
+uint64_t g_block_calls = 0;
+
+// Drops idle blocks of the device, the longest unused first, until `want` more
+// bytes fit the total: frees them in the order of s.  False when they do not.
+bool make_room(int dev, size_t want, hipStream_t s) {
+    while (g_block_bytes + want > kBlockTotal) {
+        auto oldest = g_blocks.end();
+        for (auto it = g_blocks.begin(); it != g_blocks.end(); ++it) {
+            const ScratchBlock &b = it->second;
+            if (it->first.first != dev || it->first.second == s || b.busy || !b.recorded ||
+                g_block_calls - b.last < kBlockIdle)
+                continue;
+            if (oldest == g_blocks.end() || b.last < oldest->second.last) oldest = it;
+        }
+        if (oldest == g_blocks.end()) return false;
+        ScratchBlock &b = oldest->second;
+        if (hipStreamWaitEvent(s, b.done, 0) != hipSuccess || hipFreeAsync(b.p, s) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        (void)hipEventDestroy(b.done);
+        g_block_bytes -= b.bytes;
+        g_blocks.erase(oldest);
+    }
+    return true;
+}
 
 // The stream's block, taken for the caller, or null where there is none to
 // have (the caller then allocates).
@@ -181,12 +216,13 @@ void *take_block(int dev, size_t need, hipStream_t s) {
     // (hipStreamPerThread names a different stream in every thread)
     if (need > kBlockMax || s == hipStreamPerThread) return nullptr;
     std::lock_guard<std::mutex> lock(g_block_mu);
+    ++g_block_calls;
     ScratchBlock &b = g_blocks[std::make_pair(dev, s)];
     if (b.busy) return nullptr;
     if (b.bytes < need) {
         size_t want = (size_t)1 << 20;
         while (want < need) want *= 2;
-        if (g_block_bytes - b.bytes + want > kBlockTotal) return nullptr;
+        if (!make_room(dev, want - b.bytes, s)) return nullptr;
         void *p = nullptr;
         if (hipMallocAsync(&p, want, s) != hipSuccess) {
             (void)hipGetLastError();
@@ -198,12 +234,19 @@ void *take_block(int dev, size_t need, hipStream_t s) {
         b.bytes = want;
     }
     b.busy = true;
+    b.recorded = false;
+    b.last = g_block_calls;
     return b.p;
 }
 
 void return_block(int dev, hipStream_t s) {
     std::lock_guard<std::mutex> lock(g_block_mu);
-    g_blocks[std::make_pair(dev, s)].busy = false;
+    ScratchBlock &b = g_blocks[std::make_pair(dev, s)];
+    b.busy = false;
+    if (g_block_bytes <= kBlockTotal / 2) return;
+    if (!b.done && hipEventCreateWithFlags(&b.done, hipEventDisableTiming) != hipSuccess) b.done = nullptr;
+    b.recorded = b.done && hipEventRecord(b.done, s) == hipSuccess;
+    if (!b.recorded) (void)hipGetLastError();
 }
 
 // Frees the blocks that no call holds.
@@ -217,6 +260,7 @@ void release_blocks() {
             continue;
         }
         if (it->second.p) (void)hipFree(it->second.p);
+        if (it->second.done) (void)hipEventDestroy(it->second.done);
         g_block_bytes -= it->second.bytes;
         it = g_blocks.erase(it);
     }
@@ -362,3 +406,13 @@ int set_pointer_checks(int enabled) {
 }
 
 }  // namespace gfh
+
+// Bytes kept for the current device's stream s.  Not part of the API: for the
+// tests.
+extern "C" __attribute__((visibility("default"))) size_t gfh_internal_scratch_kept(hipStream_t s) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    std::lock_guard<std::mutex> lock(gfh::g_block_mu);
+    const auto it = gfh::g_blocks.find(std::make_pair(dev, s));
+    return it == gfh::g_blocks.end() ? 0 : it->second.bytes;
+}

@@ -27,9 +27,12 @@
  *    the host before any launch; nothing is launched when a call fails.
  *  - Entry points are re-entrant.  Calls that take `workspace` use only that
  *    memory as scratch; when `workspace` is NULL they use a block kept
- *    per stream (up to 64 MB each and 256 MB in all, released by
- *    gfh_shutdown) or, beyond that, allocate stream-ordered scratch
- *    (hipMallocAsync/hipFreeAsync) on `stream`.  The *_workspace_size
+ *    per stream (up to 64 MB each and 256 MB in all) or, beyond that,
+ *    allocate stream-ordered scratch (hipMallocAsync/hipFreeAsync) on
+ *    `stream`.  A block outlives its stream: gfh_shutdown releases all of
+ *    them, and when the total is reached blocks that have not been used for a
+ *    while pass to other streams.  Let a stream's calls finish before it is
+ *    destroyed.  The *_workspace_size
  *    queries return 0 for shapes their entry point rejects as out of range.
  *  - HIP graphs: calls may be captured on a stream once the same call (same
  *    or larger sizes) has run on that stream outside a capture, with caller

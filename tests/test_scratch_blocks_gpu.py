@@ -58,3 +58,38 @@ def test_threads(torch_dev, own_streams):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_idle_blocks_pass_to_other_streams(torch_dev):
+    """Blocks that fill the total and then lie idle, as those of destroyed
+    streams do (a block does not know), go to streams that come later."""
+    import ctypes as C
+
+    import torch
+    import ghostflow_hip as gh
+    lib = C.CDLL(gh.lib()._name)
+    lib.gfh_internal_scratch_kept.restype = C.c_size_t
+    lib.gfh_internal_scratch_kept.argtypes = [C.c_void_p]
+    big, big_ref = _case(torch, torch_dev, 2100, 16384, 64, 0)  # 34 MB: a block of 64
+    small, small_ref = _case(torch, torch_dev, 100, 512, 64, 1)
+    torch.cuda.synchronize()
+    assert gh.lib().gfh_shutdown() == 0
+
+    def kept(s, args=big, ref=big_ref):
+        with torch.cuda.stream(s):
+            got = gh.qlinear_dynamic(*args)
+        s.synchronize()
+        assert torch.equal(got, ref)
+        return lib.gfh_internal_scratch_kept(s.cuda_stream) >> 20
+
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    assert [kept(s) for s in streams] == [64] * 4 + [0] * 2
+    for _ in range(300):
+        kept(streams[4], small, small_ref)
+    # blocks from half the total on record an event to wait for: two of the four
+    assert [kept(s) for s in streams[4:]] == [64] * 2
+    assert sum(lib.gfh_internal_scratch_kept(s.cuda_stream) for s in streams) <= 256 << 20
+    assert [kept(s) for s in streams[:2]] == [64] * 2
+    for s in streams:
+        kept(s)
+    assert gh.lib().gfh_shutdown() == 0
