@@ -43,7 +43,8 @@ def test_line_fields_and_size():
         assert k in line["roofline"]
     for k in ("value", "unit", "cores", "kind", "sample"):
         assert k in line["cpu_baseline"]
-    assert line["roofline"]["frac"] == round(147.3 / 157.3, 4)
+    # fp32 products are six bf16 ones: 2500 / 6 TFLOP/s bound them
+    assert line["roofline"]["peak"] == 416.7 and line["roofline"]["frac"] == round(147.3 * 6 / 2500, 4)
     # every north-star component is summarized, nothing else is
     assert sorted(line["north_star"]) == sorted(b.NORTH_STAR_COMPONENTS)
     assert line["components"]["count"] == len(b.NORTH_STAR_COMPONENTS) + 60
