@@ -68,10 +68,12 @@ constexpr int kBK = 32;  // k per stage: one 16x16x32 MFMA step
 // Geometry of a BM x BN tile on an NWM x NWN wave grid.  A stage of an
 // operand with R rows is three bf16 planes, each four chunks of 8 k: row r of
 // chunk c is 16 bytes at c * kChunk(R) + 16 r.
-template <int BM_, int BN_, int NWM_, int NWN_, bool AK_, bool BK_>
+// WIDE: leading dimensions beyond the 32-bit offsets inside a tile.
+template <int BM_, int BN_, int NWM_, int NWN_, bool AK_, bool BK_, bool WIDE_ = false>
 struct X3Geo {
     static constexpr int BM = BM_, BN = BN_, NWM = NWM_, NWN = NWN_;
     static constexpr bool AK = AK_, BK = BK_;  // operand k-contiguous in memory
+    static constexpr bool WIDE = WIDE_;
     static constexpr int NT = 64 * NWM * NWN;
     static constexpr int WM = BM / NWM, WN = BN / NWN;
     static constexpr int FM = WM / 16, FN = WN / 16;
@@ -111,8 +113,9 @@ struct X3Params {
 __device__ __forceinline__ constexpr int swz(int c) { return (c & 1 ? 14 : 0) ^ (c & 2 ? 4 : 0); }
 
 // One operand's share of a stage in registers.
-template <int R, int NT, bool KC>
+template <int R, int NT, bool KC, bool WIDE>
 struct X3Loader {
+    using Off = std::conditional_t<WIDE, uint64_t, uint32_t>;
     // A unit is 4 consecutive k of one row: one 16-byte load of a k-contiguous
     // operand (8 lanes cover a row's stage, 128 bytes), four 4-byte loads of a
     // k-major one (64 lanes on adjacent rows).
@@ -120,8 +123,8 @@ struct X3Loader {
     static constexpr int U = R * (kBK / F) / NT;
     static_assert(U >= 1 && U * NT * F == R * kBK, "whole units per thread");
     float v[U][F];
-    uint32_t off[U];  // byte offset of the unit, from one stage before the one it is loaded from
-    uint32_t at;      // where unit 0's pieces go in a plane
+    Off off[U];   // byte offset of the unit, from one stage before the one it is loaded from
+    uint32_t at;  // where unit 0's pieces go in a plane
 
     // Unit u lies kRows rows (k-contiguous) or kChunks chunks of 8 k (k-major)
     // after unit u - 1.
@@ -139,10 +142,10 @@ struct X3Loader {
             const int id = tid + u * NT;
             if (KC) {
                 const int64_t r = min((int64_t)(id / 8), rows - 1 - row0);
-                off[u] = (uint32_t)((r * ld + first_k(id) + kBK) * 4);
+                off[u] = (Off)((r * ld + first_k(id) + kBK) * 4);
             } else {
                 const int64_t r = min((int64_t)(id % R), rows - 1 - row0);
-                off[u] = (uint32_t)(((first_k(id) + kBK) * ld + r) * 4);
+                off[u] = (Off)(((first_k(id) + kBK) * ld + r) * 4);
             }
         }
     }
@@ -155,7 +158,7 @@ struct X3Loader {
     __device__ __forceinline__ void move_down(int tid, int64_t ld, int left) {
         asm volatile("" : "+v"(tid));
 #pragma unroll
-        for (int u = 0; u < U; ++u) off[u] -= (uint32_t)(moved(first_k(tid + u * NT), left) * (KC ? 1 : ld) * 4);
+        for (int u = 0; u < U; ++u) off[u] -= (Off)(moved(first_k(tid + u * NT), left) * (KC ? 1 : ld) * 4);
     }
     // Requests unit u of a stage.  `base` is one stage before it (k-contiguous:
     // the tile's first row at that k; k-major: that k row), so that the
@@ -163,6 +166,19 @@ struct X3Loader {
     // (Buffer loads: a uniform base and row offset in scalar registers, the
     // lane's offset in one vector register.)
     __device__ __forceinline__ void load(int u, const char *base, int64_t ld) {
+        if constexpr (WIDE) {
+            typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+            const float *from = reinterpret_cast<const float *>(base + off[u]);
+            if constexpr (KC) {
+                const f32x4 x = *reinterpret_cast<const f32x4_any *>(from);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[u][e] = x[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < F; ++e) v[u][e] = from[e * ld];
+            }
+            return;
+        }
         const __amdgpu_buffer_rsrc_t buf = coherent_buffer(base, 0xffffffffu);
         if constexpr (KC) {
             const f32x4 x = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, (int)off[u], 0, 0));
@@ -277,8 +293,8 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
     a_base -= a_step;
     b_base -= b_step;
 
-    X3Loader<BM, NT, G::AK> ga;
-    X3Loader<BN, NT, G::BK> gb;
+    X3Loader<BM, NT, G::AK, G::WIDE> ga;
+    X3Loader<BN, NT, G::BK, G::WIDE> gb;
     ga.init(tid, p.lda, m0, p.m);
     gb.init(tid, p.ldb, n0, p.n);
     constexpr int UA = decltype(ga)::U, UB = decltype(gb)::U;
@@ -582,14 +598,14 @@ constexpr X3Tile kTiles[] = {{256, 128, 1, 1.75, 2.20, 4.5},
                              {32, 64, 4, 0.44, 0.30, 0.3}};
 
 // Tile I of the table on an NWM x NWN wave grid, in the layout of d.
-template <int I, int NWM, int NWN>
+template <int I, int NWM, int NWN, bool WIDE = false>
 void launch_tile(const SgemmDesc &d, const X3Params &p, dim3 grid, hipStream_t s) {
     constexpr int BM = kTiles[I].bm, BN = kTiles[I].bn;
     static_assert(X3Geo<BM, BN, NWM, NWN, true, true>::kPerCu == kTiles[I].per_cu &&
                       64 * NWM * NWN == kTiles[I].threads(),
                   "the plan's figures are the kernel's");
     auto go = [&](auto ak, auto bk) {
-        hipLaunchKernelGGL((sgemm_x3_kernel<X3Geo<BM, BN, NWM, NWN, decltype(ak)::value, decltype(bk)::value>>), grid,
+        hipLaunchKernelGGL((sgemm_x3_kernel<X3Geo<BM, BN, NWM, NWN, decltype(ak)::value, decltype(bk)::value, WIDE>>), grid,
                            dim3(64 * NWM * NWN), 0, s, p);
     };
     using Y = std::true_type;
@@ -605,6 +621,15 @@ struct X3Plan {
     int slices;
 };
 
+// Whether the offsets inside a tile fit 32 bits: up to 256 rows of a
+// k-contiguous operand, 32 k and the stage before of a k-major one (and the
+// three k that the loads' scalar offsets add).
+bool x3_offsets_fit(const SgemmDesc &d) {
+    constexpr int64_t kRows = (int64_t)1 << 22, kMajor = (int64_t)1 << 23;
+    return d.lda <= (d.trans_a ? kMajor : kRows) && d.ldb <= (d.trans_b ? kRows : kMajor);
+}
+constexpr int kWideTile = 3;  // 64-bit offsets: one tile size
+
 // Work items of a launch: 32 bits.
 bool x3_grid_fits(const X3Tile &t, int64_t workgroups) { return workgroups * t.threads() < (int64_t)1 << 32; }
 
@@ -617,14 +642,15 @@ bool x3_grid_fits(const X3Tile &t, int64_t workgroups) { return workgroups * t.t
 // 20% less time over all, none more than 2% slower.)
 X3Plan plan_x3(const SgemmDesc &d, int64_t count) {
     const int64_t stages = (d.k + kBK - 1) / kBK, cus = device_cu_count();
+    const bool wide = !x3_offsets_fit(d);
     X3Plan best{0, 1};
     double least = 1e30;
     for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
         const X3Tile &t = kTiles[i];
         const int64_t tiles = t.tiles(d, count);
-        if (!x3_grid_fits(t, tiles)) continue;
+        if (!x3_grid_fits(t, tiles) || (wide && i != kWideTile)) continue;
         const int64_t round = t.per_cu * cus;
-        for (int sl = 1; sl <= 16; ++sl) {
+        for (int sl = 1; sl <= 256; sl += sl < 16 ? 1 : sl / 4) {
             const double one = (double)t.bm * t.bn * 4, part = (double)sl * (double)tiles * one;
             if (sl > 1 && (stages / sl < 4 || part > 64e6)) break;
             const int64_t tasks = tiles * sl, rem = tasks % round;
@@ -643,9 +669,8 @@ X3Plan plan_x3(const SgemmDesc &d, int64_t count) {
 }
 
 bool x3_takes(const SgemmDesc &d, int64_t count) {
-    constexpr int64_t kMaxLd = 1 << 21;
-    return d.k >= 32 && d.k <= (int64_t)1 << 30 && d.m >= 1 && d.n >= 1 && d.lda <= kMaxLd && d.ldb <= kMaxLd &&
-           x3_grid_fits(kTiles[0], kTiles[0].tiles(d, count));
+    const X3Tile &t = kTiles[x3_offsets_fit(d) ? 0 : kWideTile];
+    return d.k >= 32 && d.k <= (int64_t)1 << 30 && d.m >= 1 && d.n >= 1 && x3_grid_fits(t, t.tiles(d, count));
 }
 
 // d[0] gives the shape and layout of all products.
@@ -676,7 +701,12 @@ int launch_products(const SgemmDesc *d, X3Params &p, hipStream_t s) {
         case 0: launch_tile<0, 4, 2>(*d, p, grid, s); break;
         case 1: launch_tile<1, 2, 4>(*d, p, grid, s); break;
         case 2: launch_tile<2, 4, 2>(*d, p, grid, s); break;
-        case 3: launch_tile<3, 2, 4>(*d, p, grid, s); break;
+        case 3:
+            if (x3_offsets_fit(*d))
+                launch_tile<3, 2, 4>(*d, p, grid, s);
+            else
+                launch_tile<3, 2, 4, true>(*d, p, grid, s);
+            break;
         default: launch_tile<4, 1, 4>(*d, p, grid, s); break;
     }
     return check_launch("sgemm (bf16 pieces)");
@@ -686,9 +716,8 @@ int launch_products(const SgemmDesc *d, X3Params &p, hipStream_t s) {
 
 // Whether this kernel takes the product.  K >= 32: below that the fp32 chain
 // is short enough for its rounding to be smaller than the pieces'.  The
-// operand offsets inside a tile are 32-bit, and so is the number of threads of
-// the launch: from 2^29 rows on the smaller tiles drop out (128 x 64 has four
-// threads a row), at 2^31 the largest.
+// number of threads of the launch is 32-bit: from 2^29 rows on the smaller
+// tiles drop out (128 x 64 has four threads a row), at 2^31 the largest.
 bool sgemm_x3_fits(const SgemmDesc &d) { return x3_takes(d, std::max<int64_t>(d.batch, 1)); }
 
 int launch_sgemm_x3(const SgemmDesc &d, hipStream_t s) {

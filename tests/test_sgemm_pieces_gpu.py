@@ -226,21 +226,40 @@ def test_group_equals_separate_products(torch_dev):
     assert ((h.double() - ref).abs() <= bound).all()
 
 
-def test_offset_limits_fall_back(torch_dev):
-    """A leading dimension beyond the tile kernel's 32-bit offsets still runs."""
+@pytest.mark.parametrize("over", [0, 5])
+@pytest.mark.parametrize("operand,ta,tb", [("a", 0, 0), ("a", 0, 1), ("a", 1, 0), ("b", 0, 0), ("b", 0, 1), ("b", 1, 1)])
+def test_offset_limits(torch_dev, operand, ta, tb, over):
+    """Leading dimensions at the limits of the tiles' 32-bit offsets, 2^22 for a
+    k-contiguous operand and 2^23 for a k-major one, and just beyond, where
+    64-bit ones take their place."""
     import torch
-    gh = _gh()
-    ld, m, k, n = (1 << 21) + 8, 66, 40, 70
-    buf = torch.zeros((m - 1) * ld + k, device=torch_dev)
-    a = torch.as_strided(buf, (m, k), (ld, 1))
-    a.copy_(torch.randn(m, k, device=torch_dev))
-    b = torch.randn(k, n, device=torch_dev)
-    out = torch.empty(m, n, device=torch_dev)
-    rc = gh.lib().gfh_sgemm(0, 0, m, n, k, C.c_float(1.0), buf.data_ptr(), ld, b.data_ptr(), n, C.c_float(0.0),
-                            out.data_ptr(), n, None, torch.cuda.current_stream().cuda_stream)
+    kmajor = ta if operand == "a" else not tb
+    m, k, n = 263, 171 if kmajor else 1003, 270
+    assert plan(m, n, k, ta, tb) is not None
+    ld = (1 << (23 if kmajor else 22)) + over
+    _big_ld(torch, torch_dev, operand, m, n, k, ta, tb, ld)
+
+
+def test_offset_limit_of_the_largest_tile(torch_dev):
+    import torch
+    m, n, k = 2050, 2050, 525
+    assert plan(m, n, k)[:2] == (256, 128)
+    _big_ld(torch, torch_dev, "a", m, n, k, 0, 0, 1 << 22)
+
+
+def _big_ld(torch, dev, operand, m, n, k, ta, tb, ld):
+    def stored(rows, cols, wide):
+        w = ld if wide else cols
+        x = torch.as_strided(torch.empty((rows - 1) * w + cols, device=dev), (rows, cols), (w, 1))
+        return x.copy_(torch.randn(rows, cols, device=dev))
+
+    a = stored(*((k, m) if ta else (m, k)), operand == "a")
+    b = stored(*((n, k) if tb else (k, n)), operand == "b")
+    out = torch.empty(m, n, device=dev)
+    rc = _gh().lib().gfh_sgemm(ta, tb, m, n, k, C.c_float(1.0), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+                               C.c_float(0.0), out.data_ptr(), n, None, torch.cuda.current_stream().cuda_stream)
     assert rc == 0
-    s = a.double().abs() @ b.double().abs()
-    assert ((out.double() - a.double() @ b.double()).abs() <= (k + 4) * 2.0 ** -24 * s).all()
+    _check(torch, out, (a.t() if ta else a).contiguous(), (b.t() if tb else b).contiguous(), k)
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])

@@ -45,3 +45,12 @@ def test_shapes_of_the_gpu_tests_reach_every_tile():
     # the four layouts run the same tile
     for s, p in plans.items():
         assert {plan(*s, ta, tb) for ta in (0, 1) for tb in (0, 1)} == {p}
+
+
+def test_long_k_of_small_products_fills_the_gpu():
+    """A few tiles over a long K: enough slices for the CUs, at least four
+    stages of 32 each."""
+    for m, n, k in ((64, 64, 3000000), (100, 100, 500000), (33, 20, 8190), (33, 20, 2000)):
+        bm, bn, slices, _ = plan(m, n, k, 0, 1)
+        tiles = -(-m // bm) * -(-n // bn)
+        assert min(200, k // 32 // 8) <= slices * tiles and k // 32 // slices >= 4
