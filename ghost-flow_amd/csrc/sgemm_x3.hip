@@ -13,8 +13,8 @@
 // _bf16 per 32 k do the same product: a register-only loop of them on split
 // N(0, 1) data sustains 1920 TFLOP/s (320 of fp32 product; 1570 with the
 // 32x32x16 form) at about 1.8 GHz, the power limit.  Measured, before -> now
-// (us; NT / NN / TN): 4096^3 935 / 950 / 951 -> 594 / 598 / 618; 2048^3 NN
-// 131 -> 93; 1000 x 1500 x 784 NN 42.6 -> 24.5; 64 x 11008 x 4096 NT 90 -> 56.
+// (us; NT / NN / TN): 4096^3 938 / 956 / 959 -> 604 / 608 / 623; 2048^3 NN
+// 131 -> 93; 1000 x 1500 x 784 NN 42.6 -> 24.3; 64 x 11008 x 4096 NT 90 -> 56.
 // Relative error against 64 bits: 4096^3 1.1e-6 -> 2.2e-7, 512 x 512 x 64
 // 1.1e-7 -> 4.7e-8 (no shape of the sweep came out larger than before).
 //
@@ -371,8 +371,10 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
     for (int u = 0; u < UA; ++u) ga.store(u, ring(0));
 #pragma unroll
     for (int u = 0; u < UB; ++u) gb.store(u, ring(0) + G::kABytes);
-    before_load(1);
-    load(1);
+    if (nk > 1) {
+        before_load(1);
+        load(1);
+    }
     wait_lgkm0();
     __builtin_amdgcn_s_barrier();
     read_b(0, 0);
@@ -423,7 +425,7 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
         // moves them into the blocks after the next branch, past the
         // scheduling barriers, and every row block's sums stay in registers
         // until then (256 and 26 to 44 spilled, 1027 us at 4096^3; with this
-        // and the loop in pairs 230 and none).
+        // and the loop in pairs 226 to 246 and none).
 #pragma unroll
         for (int i = 0; i + 1 < FM; ++i)
 #pragma unroll
@@ -432,12 +434,33 @@ __global__ __launch_bounds__(G::NT, G::kWavesPerSimd) void sgemm_x3_kernel(X3Par
                 asm volatile("" : "+v"(x));
             }
     };
+    // The last stage has nothing to split, request or wait for.  (As a stage
+    // like the others it split and loaded itself once more: NN 64 x 64 x
+    // 3000000 483 us instead of 406, 96 x [500, 64] x [64, 500] 41.1 instead
+    // of 38.9, 4096^3 618 instead of 604.)
+    auto last = [&](auto par) __attribute__((always_inline)) {
+        constexpr int P = decltype(par)::value;
+        unrolled<FM>([&](auto rc) __attribute__((always_inline)) {
+            constexpr int r = decltype(rc)::value;
+            if constexpr (r + 1 < FM) read_a((r + 1) & 1, P, r + 1);
+#pragma unroll
+            for (int s = 0; s < 6; ++s) step(r, s, r & 1, P);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    using Even = std::integral_constant<int, 0>;
+    using Odd = std::integral_constant<int, 1>;
     int t = 0;
-    for (; t + 1 < nk; t += 2) {
-        stage(t, std::integral_constant<int, 0>{});
-        stage(t + 1, std::integral_constant<int, 1>{});
+    for (; t + 2 < nk; t += 2) {
+        stage(t, Even{});
+        stage(t + 1, Odd{});
     }
-    if (t < nk) stage(t, std::integral_constant<int, 0>{});
+    if (t + 1 < nk) {
+        stage(t, Even{});
+        last(Odd{});
+    } else {
+        last(Even{});
+    }
 #pragma unroll
     for (int j = 0; j < FN; ++j) add_sum(FM - 1, j);
 
