@@ -54,8 +54,8 @@ namespace gfh {
 namespace {
 
 constexpr int kKeys = 32;      // keys per tile: one 16x16x32 MFMA step of P.V
-constexpr int kWaves = 8;
-constexpr int kThreads = 64 * kWaves;
+constexpr int kWaves = 8;     // per workgroup; kFewWaves for launches of few queries
+constexpr int kFewWaves = 4;
 
 struct X3Attn {
     const float *q, *k, *v;
@@ -79,8 +79,9 @@ __device__ __forceinline__ int swz(int c) { return (c & 1 ? 14 : 0) ^ (c & 2 ? 4
 // key r at r ^ swz(c) ^ u of its 16-key block (16 bytes each).  V: plane,
 // key chunk c (keys 4c .. 4c + 3, 16 + 4c .. 16 + 4c + 3), dim r at
 // r ^ swz(c) of its 16-dim block.
-template <int DP>
+template <int DP, int NW = kWaves>
 struct Tile {
+    static constexpr int kThreads = 64 * NW;
     static constexpr int NU = DP / 32, NB = DP / 16;
     static constexpr int kPlane = kKeys * DP * 2;
     static constexpr int kBuf = 3 * kPlane;  // one tile of K or V
@@ -90,9 +91,10 @@ struct Tile {
 };
 
 // A thread's share of a K/V tile in registers.
-template <int DP>
+template <int DP, int NW>
 struct KvRegs {
-    using T = Tile<DP>;
+    using T = Tile<DP, NW>;
+    static constexpr int kThreads = T::kThreads;
     float k[T::U][4], v[T::U][4];
 
     __device__ __forceinline__ void load(const X3Attn &p, const float *K, const float *V, int k0, int tid) {
@@ -279,12 +281,15 @@ __device__ __forceinline__ void set_f32(const X3Attn &p, const float *Q, const f
     }
 }
 
-template <int DP, int SETS, bool CAUSAL, bool MASK, bool WEIGHTS>
-__global__ __launch_bounds__(kThreads, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_x3_kernel(X3Attn p) {
-    using T = Tile<DP>;
+// NW = kFewWaves: four waves and one V buffer, so that two workgroups share a
+// CU at D > 64 (launch_sdpa_x3 has the rule).
+template <int DP, int SETS, bool CAUSAL, bool MASK, bool WEIGHTS, int NW>
+__global__ __launch_bounds__(64 * NW, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_x3_kernel(X3Attn p) {
+    using T = Tile<DP, NW>;
     constexpr int NU = T::NU, NB = T::NB;
-    constexpr int kQ = 16 * SETS * kWaves;  // queries per workgroup
-    __shared__ __attribute__((aligned(1024))) char lds[5 * T::kBuf];  // K, K, V, V, V
+    constexpr bool FEW = NW < kWaves;
+    constexpr int kQ = 16 * SETS * NW;  // queries per workgroup
+    __shared__ __attribute__((aligned(1024))) char lds[(FEW ? 3 : 5) * T::kBuf];  // K, K, V (, V, V)
     char *const ldsv = lds + 2 * T::kBuf;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -298,7 +303,7 @@ __global__ __launch_bounds__(kThreads, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_
     const int blk = CAUSAL ? (int)gridDim.y - 1 - (int)blockIdx.y : (int)blockIdx.y;  // heaviest first
     const int wq0 = blk * kQ + wave * 16 * SETS;  // this wave's first query
 
-    KvRegs<DP> kv;
+    KvRegs<DP, NW> kv;
     kv.load(p, K, V, 0, tid);
     // (lanes that met an element beyond the pieces; a scale this large could
     // raise scores out of the pieces' last bits)
@@ -460,11 +465,11 @@ __global__ __launch_bounds__(kThreads, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_
         }
     };
 
-    const bool late = wave >= kWaves / 2;
+    const bool late = !FEW && wave >= NW / 2;
     bool pending = false;
     int vc = 0, vp = 2;  // V buffers of this tile and the one before
     for (int t = 0; t < ntiles; ++t) {
-        const int k0 = t * kKeys, vn = vc == 2 ? 0 : vc + 1;
+        const int k0 = t * kKeys, vn = FEW || vc == 2 ? 0 : vc + 1;
         if (pending) weigh(ldsv + vp * T::kBuf);
         pending = false;
         if (live && k0 < wave_end && any_kept()) {
@@ -483,7 +488,12 @@ __global__ __launch_bounds__(kThreads, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_
 #pragma unroll
         for (int u = 0; u < T::U; ++u) {
             kv.store_k(u, lds + ((t + 1) & 1) * T::kBuf, tid);
-            kv.store_v(u, ldsv + vn * T::kBuf, tid);
+            if (!FEW) kv.store_v(u, ldsv + vn * T::kBuf, tid);
+        }
+        if constexpr (FEW) {
+            __syncthreads();  // every wave is done with this tile's V
+#pragma unroll
+            for (int u = 0; u < T::U; ++u) kv.store_v(u, ldsv, tid);
         }
         kv.load(p, K, V, k0 + 2 * kKeys, tid);
         __syncthreads();
@@ -585,13 +595,13 @@ __global__ __launch_bounds__(kThreads, SETS == 1 && DP <= 64 ? 4 : 2) void sdpa_
     }
 }
 
-template <int DP, int SETS>
+template <int DP, int SETS, int NW = kWaves>
 void launch_d(const X3Attn &p, int64_t bh, bool causal, hipStream_t s) {
-    const dim3 grid((unsigned)bh, (unsigned)((p.sq + 16 * SETS * kWaves - 1) / (16 * SETS * kWaves)));
+    const dim3 grid((unsigned)bh, (unsigned)((p.sq + 16 * SETS * NW - 1) / (16 * SETS * NW)));
     const bool mask = p.mask != nullptr, weights = p.weights != nullptr;
     auto go = [&](auto cc, auto mc, auto wc) {
-        hipLaunchKernelGGL((sdpa_x3_kernel<DP, SETS, decltype(cc)::value, decltype(mc)::value, decltype(wc)::value>), grid,
-                           dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((sdpa_x3_kernel<DP, SETS, decltype(cc)::value, decltype(mc)::value, decltype(wc)::value, NW>),
+                           grid, dim3(64 * NW), 0, s, p);
     };
     using Y = std::true_type;
     using N = std::false_type;
@@ -645,13 +655,23 @@ int launch_sdpa_x3(const SdpaDesc &d, hipStream_t s) {
     p.scale = d.scale;
     const int64_t bh = d.b * d.h;
     // Two sets per wave halve the tile splits and fragment reads per query;
-    // they pay where the launch still holds two rounds of workgroups and the
-    // sets' registers leave no second workgroup per CU anyway (us, two sets /
-    // one: B = 4, H = 32 causal, D = 128, S = 512 77 / 63, 1000 187 / 204,
-    // 2048 673 / 760; D = 80, S = 1000 139 / 156; D = 64, S = 1000 105 / 99;
-    // with weights 2 x 8 x 1000, D = 128 248 / 147).
-    const bool two = d.d > 64 && !d.weights && bh * ((d.sq + 255) / 256) >= 512;
-    if (d.d <= 32)
+    // they pay where the launch still holds two rounds of workgroups, the
+    // second set is not empty, and the sets' registers leave no second
+    // workgroup per CU anyway (us, two sets / one: B = 4, H = 32 causal, D =
+    // 128, S = 512 77 / 63, 1000 187 / 204, 2048 673 / 760; D = 80, S = 1000
+    // 139 / 156; D = 64, S = 1000 105 / 99; with weights 2 x 8 x 1000, D = 128
+    // 248 / 147; 2048 slices of 128 queries and 700 keys, D = 96 509 / 486).
+    const bool two = d.d > 64 && !d.weights && d.sq > 128 && bh * ((d.sq + 255) / 256) >= 512;
+    // Few queries leave most waves of a workgroup with tiles to split and
+    // nothing to multiply; at D > 64 its LDS also fills the CU.  With four
+    // waves and one V buffer two share it: worth it once there are more
+    // workgroups than CUs (us, four waves / eight: 2048 slices, 700 keys, D =
+    // 96, 1 query 201 / 281, 64 queries 294 / 344, 80 502 / 403; 600 slices,
+    // D = 128, 1 query 111 / 119; 200 slices 49 / 40).
+    const bool few = d.d > 64 && d.sq <= 16 * kFewWaves && bh > device_cu_count();
+    if (few)
+        d.d <= 96 ? launch_d<96, 1, kFewWaves>(p, bh, d.causal, s) : launch_d<128, 1, kFewWaves>(p, bh, d.causal, s);
+    else if (d.d <= 32)
         launch_d<32, 1>(p, bh, d.causal, s);
     else if (d.d <= 64)
         launch_d<64, 1>(p, bh, d.causal, s);

@@ -103,6 +103,16 @@ def test_two_sets_per_wave(torch_dev, d, causal, kind):
     _check(torch, torch_dev, 4, 43, 530, 530, d, causal, kind, False)
 
 
+@pytest.mark.parametrize("d", [72, 96, 128])
+@pytest.mark.parametrize("sq,skv", [(1, 1), (1, 300), (16, 33), (17, 95), (64, 130), (65, 64)])
+def test_few_queries_many_slices(torch_dev, sq, skv, d):
+    """More slices than CUs: up to 64 queries run on workgroups of four waves."""
+    import torch
+    _check(torch, torch_dev, 2, 131, sq, skv, d, False, "none", False)
+    _check(torch, torch_dev, 2, 131, sq, skv, d, False, "odd", True)
+    _check(torch, torch_dev, 131, 2, sq, sq, d, True, "none", sq % 2 == 0)
+
+
 @pytest.mark.parametrize("d", [20, 64, 128])
 def test_wide_ranges(torch_dev, d):
     """Large logits, small and large values, and elements beyond the pieces
