@@ -11,12 +11,12 @@
 //   out = attn . Wo^T + bo
 //
 // The projections are launch_sgemm NT calls (the row-dot GEMV up to 4 rows,
-// the skinny MFMA GEMM up to 64, the MFMA tile GEMM beyond), with q, k and v
-// in one grouped launch up to 64 rows when their shapes agree.  Attention reads q, K and V in the
-// [B, S, E] layout where head h is a block of columns -- the storage of the
-// reference's reshape_for_attention view (:146-150) -- with the decode
-// kernel (kv_attention.hip) for up to 16 queries and the tiled SDPA kernel
-// (attention.hip, strided) beyond; its output lands directly in the merged
+// the skinny MFMA GEMM up to 32, the tiles on bf16 pieces beyond), with q, k
+// and v in one grouped launch when their shapes agree.  Attention reads q, K
+// and V in the [B, S, E] layout where head h is a block of columns -- the
+// storage of the reference's reshape_for_attention view (:146-150) -- with the
+// decode kernel (kv_attention.hip) for up to 16 queries and the SDPA kernel
+// (attention_x3.hip, strided) beyond; its output lands directly in the merged
 // [B, S, E] order that reshape_from_attention (:152-157) produces.
 #include <algorithm>
 
@@ -82,8 +82,16 @@ int launch_mha_forward(const MhaDesc &d, void *workspace, hipStream_t s) {
     const int nproj = d.sk > 0 ? 3 : 1;
     // Where query, key and value have the same rows the three projections
     // share one launch: 3x the columns fill the GPU better than one projection
-    // does, and two launch tails go away.
-    if (sgemm_nt_group_fits(proj, nproj)) {
+    // does, and two launch tails go away.  (Not where an input lies inside a
+    // cache: another projection would write it while it is read.)
+    const int64_t cached = d.b * d.capacity * e;
+    auto inside = [&](const float *x, int64_t rows) {
+        auto meets = [&](const float *c) { return x < c + cached && c < x + rows * e; };
+        return meets(d.k_cache) || meets(d.v_cache);
+    };
+    const bool apart =
+        d.sk == 0 || !(inside(d.query, d.b * d.sq) || inside(d.key, d.b * d.sk) || inside(d.value, d.b * d.sk));
+    if (apart && sgemm_nt_group_fits(proj, nproj)) {
         GFH_TRY(launch_sgemm_nt_group(proj, nproj, s));
     } else {
         for (int i = 0; i < nproj; ++i) GFH_TRY(launch_sgemm(proj[i], s));

@@ -222,3 +222,29 @@ def test_projections_equal_separate_linears(torch_dev, b, sq, sk, p, exact):
         assert torch.equal(out, ref)
     else:
         assert_rel(to_np(out), to_np(ref).astype(np.float64))
+
+
+@pytest.mark.parametrize("sq", [3, 20, 100])
+def test_query_inside_the_cache(torch_dev, sq):
+    """A query that lies where the new values (or keys) go is projected before
+    they are written."""
+    import torch
+    gh = _gh()
+    e, h, p = 128, 2, 5
+    wq, bq, wk, bk, wv, bv, wo, bo = _dev(_params(e, 3), torch_dev)
+    q, k, v = (torch.randn(1, sq, e, device=torch_dev) for _ in range(3))
+    past = [torch.randn(1, p, e, device=torch_dev) for _ in range(2)]
+    pad = torch.zeros(1, sq, e, device=torch_dev)
+
+    def run(where):
+        kc, vc = (torch.cat([t, pad], 1) for t in past)
+        x = q
+        if where is not None:
+            x = (kc, vc)[where][:, p:]
+            x.copy_(q)
+        return gh.mha_forward_cached(x, k, v, wq, bq, wk, bk, wv, bv, wo, bo, h, kc, vc, p), kc, vc
+
+    ref = run(None)
+    for where in (0, 1):
+        for got, want in zip(run(where), ref):
+            torch.testing.assert_close(got, want, rtol=0, atol=1e-4)
