@@ -23,13 +23,15 @@
 //    iteration later, so that the softmax (VALU) of one wave of a SIMD meets
 //    the products (MFMA) of the other instead of its softmax.
 //
-// What bounds it: the six-fold products (B = 4, H = 32, S = 1000, D = 128
-// causal: 17 GFLOP of pieces per 1e9 scores, 2/3 of the matrix rate inside
-// the product phases) and, between them, splitting each tile of K and V,
-// which every workgroup repeats for its own queries.  us on f32 MFMAs ->
-// here, B = 4, H = 32: D = 128 causal S = 512 92 -> 74, 1000 303 -> 192,
-// 2048 1143 -> 681, not causal 1000 540 -> 314; D = 64 causal 165 -> 103;
-// with weights and a mask B = 4, H = 16, S = 512, D = 64 201 -> 57.
+// What bounds it: the six-fold products (3.1 TFLOP of pieces per 1e9 scores at
+// D = 128) and, between them, the softmax and splitting each tile of K and V,
+// which every workgroup repeats for its own queries: B = 4, H = 32, D = 128
+// causal the MFMAs are busy 30 / 36 / 50% of the cycles at S = 512 / 1000 /
+// 2048, VALU issue takes another 25% at S = 1000.  us on f32 MFMAs -> here, B =
+// 4, H = 32: D = 128 causal S = 512 92 -> 74, 1000 303 -> 200, 2048 1143 -> 705,
+// not causal 1000 540 -> 316; D = 64 causal 165 -> 103; with weights and a mask
+// B = 4, H = 16, S = 512, D = 64 201 -> 57.  The two-set forms of D = 128 spill
+// 2 to 26 registers.
 //
 // V and the probabilities are scaled by 2^16 before they are split (and the
 // sums scaled back), so that small ones keep their 24 bits: a weight of 2^-120
@@ -40,6 +42,8 @@
 // Inputs beyond the pieces: a workgroup that meets an element of Q, K or V
 // that is not finite or above 2^60, or a scale above 2^20, and a wave whose
 // result is not finite redo their queries on f32 MFMAs (set_f32).
+// (Bounds of buffers: the loads of a tile's last keys rely on a raw buffer
+// load returning zero where voffset + soffset passes num_records.)
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -211,7 +215,9 @@ __device__ __forceinline__ void scores(const char *lds, const bf16x8 (&qf)[SETS]
 }
 
 // f32 attention of one 16-query set straight from memory, for inputs the
-// pieces cannot carry: about ten times the time of the pieces.
+// pieces cannot carry: seven to nine times the time of the pieces (B = 4, H =
+// 32, S = 1000, D = 128 causal 244 us, with one element beyond in one head 1659,
+// in all 2192).
 template <int DP, bool CAUSAL, bool MASK, bool WEIGHTS>
 __device__ __forceinline__ void set_f32(const X3Attn &p, const float *Q, const float *K, const float *V, float *O,
                                         int64_t wrow0, int q0, int lane) {
