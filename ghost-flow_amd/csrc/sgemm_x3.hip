@@ -660,13 +660,20 @@ bool x3_grid_fits(const X3Tile &t, int64_t workgroups) { return workgroups * t.t
 // The tile and K split with the shortest estimated time for `count` products
 // of one shape: workgroups in rounds of per_cu on every CU.  K slices add the
 // partial tiles' stores, at 6 TB/s, and the last arriver's reads of a tile's
-// partials, which one workgroup takes in at 100 GB/s.  (A batch splits like a
+// partials, which one workgroup takes in at 100 GB/s.  The operands arrive no
+// faster than 5 TB/s, nor than the resident workgroups' two requested stages
+// per 3 us: with few rows one workgroup per CU keeps too little in flight (NT
+// 33 x 4096 x 4096 in 4 slices 30.1 us, in 8 26.3; of 85 products of 33-1500
+// rows whose operands lie beyond the MALL the choice is 3.6% slower than the
+// fastest on average and 28% at worst, 4.2% without this, and up to 128 rows
+// 2.4 for 3.9).  (A batch splits like a
 // group: a few slices of a long K otherwise leave most CUs idle, 2 x [4096,
 // 4096] x [4096, 64] 84 us, split 44; 29 batches of 2-64 with K 281-7981:
 // 20% less time over all, none more than 2% slower.)
 X3Plan plan_x3(const SgemmDesc &d, int64_t count) {
     const int64_t stages = (d.k + kBK - 1) / kBK, cus = device_cu_count();
     const bool wide = !x3_offsets_fit(d);
+    const double operands = 4.0 * (double)d.k * (double)(d.m + d.n) * (double)count;
     X3Plan best{0, 1};
     double least = 1e30;
     for (int i = 0; i < (int)(sizeof kTiles / sizeof kTiles[0]); ++i) {
@@ -682,6 +689,8 @@ X3Plan plan_x3(const SgemmDesc &d, int64_t count) {
             auto shared = [&](double n) { return std::max(st * t.alone, n * st * t.full) + n * t.ends; };
             double us = (double)(tasks / round) * shared(t.per_cu);
             if (rem) us += 4 * rem <= 3 * cus ? st * t.alone + t.ends : shared((double)((rem + cus - 1) / cus));
+            const double flight = (double)std::min(tasks, round) * 2 * (t.bm + t.bn) * kBK * 4;
+            us = std::max(us, operands / std::min(5e6, flight / 3));
             if (sl > 1) us += 2.5 + part / 6e6 + sl * one / 1e5;
             if (us < least) {
                 least = us;
